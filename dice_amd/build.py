@@ -27,6 +27,8 @@ SOURCES = [
     "grouped_gemm_f32.hip",
     "grouped_gemm_bf16.hip",
     "grouped_gemm_f16.hip",
+    "grouped_gemm_stream.hip",
+    "grouped_gemm_stream_f16.hip",
     "grouped_gemm_persist.hip",
     "grouped_gemm_persist_f16.hip",
     "grouped_gemm_persist_f8.hip",

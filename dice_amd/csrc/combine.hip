@@ -17,7 +17,7 @@
 // models.py:519; b = token / tokens_per_sample), applied to the fp32 sum before
 // the one rounding: two more reads per element instead of the reference's two
 // extra elementwise kernels over [N, D].
-#include "common.h"
+#include "gemm_common.h"
 
 namespace dice {
 namespace {
@@ -44,6 +44,25 @@ template <> struct Pack<f16_t> {
 
 constexpr int kMaxTopK = 8;
 
+// Chunk `i` (16 bytes of T) of a row that an fc2 launch cut along k has left as
+// `pieces` fp32 partial rows, `stride` chunks apart: their sum, in piece order,
+// rounded to T as the row of an uncut launch is.
+template <typename T>
+__device__ __forceinline__ Pack<T> sum_pieces(const void *rows, int64_t i, int pieces, int64_t stride) {
+  constexpr int V = Pack<T>::kN / 4;
+  const f32x4_t *src = (const f32x4_t *)rows + i * V;
+  f32x4_t v[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) v[q] = src[q];
+  for (int p = 1; p < pieces; ++p)
+#pragma unroll
+    for (int q = 0; q < V; ++q) v[q] += src[p * stride * V + q];
+  Pack<T> r;
+#pragma unroll
+  for (int e = 0; e < Pack<T>::kN; ++e) r.set(e, v[e / 4][e % 4]);
+  return r;
+}
+
 // What one routing slot of a token contributes: its weight and where its row
 // comes from (the cache, the slot rows, or nowhere: a zero row).
 template <typename T>
@@ -51,6 +70,7 @@ struct SlotSource {
   float w;
   const Pack<T> *row;   // nullptr: a zero row
   bool put;             // the row also goes to cache_out
+  bool cached;          // the row is the cache's
 };
 template <typename T>
 __device__ __forceinline__ SlotSource<T> slot_source(
@@ -63,6 +83,7 @@ __device__ __forceinline__ SlotSource<T> slot_source(
   if (skipped && cache_in) {
     r.row = cache_in + chunk_of_token;
     r.put = false;
+    r.cached = true;
   } else {
     // A slot the dispatch left out (masked, or an expert id outside the
     // table: inv_perm = -1) contributes a zero row, as the zero-initialised
@@ -70,6 +91,7 @@ __device__ __forceinline__ SlotSource<T> slot_source(
     const int64_t src = inv_perm ? (int64_t)inv_perm[s] : s;
     r.row = src >= 0 ? slot_out + src * vec_per_row + c : nullptr;
     r.put = skipped && have_cache_out;
+    r.cached = false;
   }
   return r;
 }
@@ -78,14 +100,16 @@ __device__ __forceinline__ SlotSource<T> slot_source(
 // first, then all K rows are requested, then they are added in slot order (two
 // memory round trips per thread instead of two per slot; same arithmetic).
 // K = 0: any top_k, slot by slot.
-template <typename T, int K>
+// SPLIT (K > 0): slot_out and / or shared_out hold partial rows (sum_pieces); reading
+// them here saves the launch that would add them up and a round trip of the rows.
+template <typename T, int K, bool SPLIT = false>
 __global__ __launch_bounds__(256) void combine_kernel(
     const Pack<T> *__restrict__ slot_out, const int32_t *__restrict__ inv_perm,
     const float *__restrict__ topk_weight, const Pack<T> *__restrict__ shared_out,
     const uint8_t *__restrict__ skip_mask, const Pack<T> *__restrict__ cache_in,
     Pack<T> *__restrict__ cache_out, Pack<T> *__restrict__ y, int64_t n_tokens, int top_k,
     int vec_per_row, const Pack<T> *__restrict__ resid, const Pack<T> *__restrict__ gate,
-    int64_t tokens_per_sample) {
+    int64_t tokens_per_sample, int slot_pieces, int64_t slot_stride, int shared_pieces) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_tokens * vec_per_row) return;
   const int64_t t = i / vec_per_row;
@@ -96,7 +120,10 @@ __global__ __launch_bounds__(256) void combine_kernel(
   // (the rows that do not depend on the routing tables are requested first, so
   // that they travel while the slot rows' addresses are still being looked up)
   Pack<T> sh{}, res{}, gt{};
-  if (shared_out) sh = shared_out[i];
+  if (shared_out) {
+    if (SPLIT && shared_pieces > 1) sh = sum_pieces<T>(shared_out, i, shared_pieces, n_tokens * vec_per_row);
+    else sh = shared_out[i];
+  }
   if (resid) {
     res = resid[i];
     gt = gate[(t / tokens_per_sample) * vec_per_row + c];
@@ -111,7 +138,9 @@ __global__ __launch_bounds__(256) void combine_kernel(
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       row[j] = Pack<T>{};
-      if (src[j].row) row[j] = *src[j].row;
+      if (SPLIT && slot_pieces > 1 && src[j].row && !src[j].cached)
+        row[j] = sum_pieces<T>(slot_out, src[j].row - slot_out, slot_pieces, slot_stride);
+      else if (src[j].row) row[j] = *src[j].row;
     }
 #pragma unroll
     for (int j = 0; j < K; ++j) {
@@ -148,15 +177,29 @@ template <typename T>
 int launch_combine(const void *slot_out, const int32_t *inv_perm, const float *w,
                    const void *shared_out, const uint8_t *skip, const void *cache_in,
                    void *cache_out, void *y, int64_t n_tokens, int top_k, int hidden,
-                   const void *resid, const void *gate, int64_t tokens_per_sample, hipStream_t s) {
+                   const void *resid, const void *gate, int64_t tokens_per_sample, hipStream_t s,
+                   int slot_pieces, int64_t slot_rows, int shared_pieces) {
   const int vec_per_row = hidden / Pack<T>::kN;
   const int64_t total = n_tokens * vec_per_row;
   const int64_t blocks = (total + 255) / 256;
-#define DICE_COMBINE_LAUNCH(K)                                                                      \
-  hipLaunchKernelGGL((combine_kernel<T, K>), dim3((unsigned)blocks), dim3(256), 0, s,               \
+  const bool split = slot_pieces > 1 || shared_pieces > 1;
+#define DICE_COMBINE_LAUNCH(K, ...)                                                                 \
+  hipLaunchKernelGGL((combine_kernel<T, K, ##__VA_ARGS__>), dim3((unsigned)blocks), dim3(256), 0, s, \
                      (const Pack<T> *)slot_out, inv_perm, w, (const Pack<T> *)shared_out, skip,     \
                      (const Pack<T> *)cache_in, (Pack<T> *)cache_out, (Pack<T> *)y, n_tokens, top_k, \
-                     vec_per_row, (const Pack<T> *)resid, (const Pack<T> *)gate, tokens_per_sample)
+                     vec_per_row, (const Pack<T> *)resid, (const Pack<T> *)gate, tokens_per_sample, slot_pieces, \
+                     slot_rows * vec_per_row, shared_pieces)
+  if constexpr (Pack<T>::kN == 8) {
+    if (split) {
+      switch (top_k) {
+        case 1: DICE_COMBINE_LAUNCH(1, true); break;
+        case 2: DICE_COMBINE_LAUNCH(2, true); break;
+        case 4: DICE_COMBINE_LAUNCH(4, true); break;
+        default: return fail(DICE_ERR_UNSUPPORTED, "dice_combine: partial rows with top_k %d", top_k);
+      }
+      return launch_status("dice_combine");
+    }
+  }
   switch (top_k) {
     case 1: DICE_COMBINE_LAUNCH(1); break;
     case 2: DICE_COMBINE_LAUNCH(2); break;
@@ -172,7 +215,8 @@ int launch_combine(const void *slot_out, const int32_t *inv_perm, const float *w
 int combine_impl(const void *slot_out, const int32_t *inv_perm, const float *topk_weight,
                  const void *shared_out, const uint8_t *skip_mask, const void *cache_in, void *cache_out,
                  void *y, int dtype, int64_t n_tokens, int top_k, int hidden, const void *resid,
-                 const void *gate, int64_t tokens_per_sample, void *stream) {
+                 const void *gate, int64_t tokens_per_sample, void *stream, int slot_pieces, int64_t slot_rows,
+                 int shared_pieces) {
   DICE_REQUIRE(slot_out && topk_weight && y, DICE_ERR_BAD_ARG, "dice_combine: null pointer");
   DICE_REQUIRE(top_k >= 1 && top_k <= kMaxTopK, DICE_ERR_BAD_ARG, "dice_combine: top_k %d outside [1, %d]",
                top_k, kMaxTopK);
@@ -192,13 +236,16 @@ int combine_impl(const void *slot_out, const int32_t *inv_perm, const float *top
   switch (dtype) {
     case DICE_F32:
       return launch_combine<float>(slot_out, inv_perm, topk_weight, shared_out, skip_mask, cache_in,
-                                   cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s);
+                                   cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s,
+                                   slot_pieces, slot_rows, shared_pieces);
     case DICE_BF16:
       return launch_combine<bf16_t>(slot_out, inv_perm, topk_weight, shared_out, skip_mask, cache_in,
-                                    cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s);
+                                    cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s,
+                                   slot_pieces, slot_rows, shared_pieces);
     case DICE_F16:
       return launch_combine<f16_t>(slot_out, inv_perm, topk_weight, shared_out, skip_mask, cache_in,
-                                   cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s);
+                                   cache_out, y, n_tokens, top_k, hidden, resid, gate, tokens_per_sample, s,
+                                   slot_pieces, slot_rows, shared_pieces);
   }
   return fail(DICE_ERR_UNSUPPORTED, "dice_combine: dtype %d", dtype);
 }

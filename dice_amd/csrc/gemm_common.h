@@ -199,6 +199,7 @@ int persist_slim_choice(int mode);  // tuning hook state: 128-row weight tiles f
 int shared_fc2_launch_choice();   // tuning hook state: 1 = the shared expert's fc2 as a launch of its own, -1 = never, 0 = by size
 bool persist_split_allowed();      // tuning hook state: fc2 launches of the layer call may cut their last turn along k
 bool route_in_prologue_allowed();   // tuning hook state: the modulated layer call may route inside its prologue kernel
+int stream_choice();               // tuning hook state: 1 = the layer call takes the streaming kernels wherever they apply, -1 = never, 0 = by size
 bool gemm_config_is_default(int mode);  // tuning hook state: nothing is set for this stage
 bool gemm_config_allows_persistent(int mode);  // tuning hook state: no tiling of the permutation-addressed kernels is forced for this stage
 int launch_grouped_gemm_persist(const PersistBatch &b, int mode, hipStream_t s);      // bf16
@@ -206,6 +207,19 @@ int launch_grouped_gemm_persist_f16(const PersistBatch &b, int mode, hipStream_t
 // fp8 activations (a_scale) and weights (w_scale) on the fp8 matrix pipe, bf16 output
 bool persist_f8_supported(const PersistBatch &b, int mode);
 int launch_grouped_gemm_persist_f8(const PersistBatch &b, int mode, hipStream_t s);
+
+// Up to two problems of a launch of the streaming kernels (grouped_gemm_stream.hip).
+struct StreamBatch {
+  int n_problems;
+  PersistProblem prob[2];
+  // fc2: pieces a problem's k range is cut into.  With more than one the kernel writes
+  // fp32 partial rows: piece i of row r at c + (i * max_rows + r) * ldc floats.
+  int pieces[2];
+  bool tall;   // 192-row tiles instead of 128-row ones
+};
+bool stream_supported(const StreamBatch &b, int mode);
+int launch_grouped_gemm_stream(const StreamBatch &b, int mode, hipStream_t s);
+int launch_grouped_gemm_stream_f16(const StreamBatch &b, int mode, hipStream_t s);
 
 // Few rows per group (at most 128 on average): a 256-row tile of the persistent
 // kernels is then mostly padding - its matrix-pipe time is that of a full tile -
@@ -228,10 +242,13 @@ int ln_modulate_route_impl(const void *x, const void *shift, const void *scale, 
                            int64_t n_tokens, int hidden, int64_t tokens_per_sample, float eps, const void *gate_w,
                            const float *gate_bias, int n_experts, int top_k, int norm_topk_prob, int32_t *topk_idx,
                            float *topk_weight, void *stream);
+// slot_pieces / shared_pieces > 1: the rows are fp32 partial rows that add up to a row (piece i of the slot rows
+// lies i * slot_rows rows on, of the shared rows i * n_tokens rows); 16-bit types, top_k 1, 2 or 4.
 int combine_impl(const void *slot_out, const int32_t *inv_perm, const float *topk_weight,
                  const void *shared_out, const uint8_t *skip_mask, const void *cache_in, void *cache_out,
                  void *y, int dtype, int64_t n_tokens, int top_k, int hidden, const void *resid,
-                 const void *gate, int64_t tokens_per_sample, void *stream);
+                 const void *gate, int64_t tokens_per_sample, void *stream, int slot_pieces = 1,
+                 int64_t slot_rows = 0, int shared_pieces = 1);
 
 int dispatch_impl(const int32_t *flat_idx, const uint8_t *skip_mask, int64_t n_slots, int n_experts,
                   int32_t *counts, int32_t *offsets, int32_t *perm, int32_t *inv_perm, void *workspace,

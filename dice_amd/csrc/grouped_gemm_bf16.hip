@@ -423,6 +423,12 @@ int persist_slim_choice(int mode) {
 bool persist_split_allowed() { return g_cfg_fc2 != 50; }
 int shared_fc2_launch_choice() { return g_cfg_fc2 == 51 ? 1 : g_cfg_fc2 == 52 ? -1 : 0; }
 bool route_in_prologue_allowed() { return g_cfg_fc1 != 50; }
+int stream_choice() {
+  if (g_cfg_fc1 == 57) return 1;
+  // (values that only choose between forms of the persistent launches leave the rule alone)
+  const bool fc1_free = g_cfg_fc1 == 0 || g_cfg_fc1 == 54 || g_cfg_fc1 == 55, fc2_free = g_cfg_fc2 == 0 || g_cfg_fc2 == 51;
+  return fc1_free && fc2_free ? 0 : -1;
+}
 bool gemm_config_is_default(int mode) { return (mode == kFc2 ? g_cfg_fc2 : g_cfg_fc1) == 0; }
 }  // namespace dice
 
@@ -439,7 +445,9 @@ bool gemm_config_is_default(int mode) { return (mode == kFc2 ? g_cfg_fc2 : g_cfg
 // the shared expert's fc2 on its own always / never (by default it does for small
 // batches, where both launches then cut their tiles along k); 54 / 55 (either stage)
 // have launches that can take 128-row weight tiles do so always / never (by default
-// where the host's model says they shorten the launch).  Any value from 20 on also keeps a
+// where the host's model says they shorten the launch); 57 (fc1) has the layer call take
+// the streaming kernels wherever they apply (by default for small batches, also under
+// fc1 = 54 / 55 and fc2 = 51; any other value of either stage keeps it off them).  Any value from 20 on also keeps a
 // dice_grouped_mlp stage whose groups average at most 128 rows on the persistent
 // kernels (21 does only that; by default such a stage takes this file's 64-row
 // tiles).  1 .. 4 name a tiling of this file's kernels for

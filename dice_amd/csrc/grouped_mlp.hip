@@ -1,4 +1,7 @@
 // C entry points of the expert MLP and of the whole layer.
+#include <cmath>
+#include <utility>
+
 #include "gemm_common.h"
 
 namespace dice {
@@ -16,6 +19,30 @@ bool is_16bit(int dtype) { return dtype == DICE_BF16 || dtype == DICE_F16; }
 int launch_persist(const PersistBatch &b, int mode, int act_dtype, hipStream_t s) {
   return act_dtype == DICE_F16 ? launch_grouped_gemm_persist_f16(b, mode, s)
                                : launch_grouped_gemm_persist(b, mode, s);
+}
+
+int launch_stream(const StreamBatch &b, int mode, int act_dtype, hipStream_t s) {
+  return act_dtype == DICE_F16 ? launch_grouped_gemm_stream_f16(b, mode, s) : launch_grouped_gemm_stream(b, mode, s);
+}
+
+// Rows of the fuller experts under a uniform routing (1.5 standard deviations).
+double rows_of_full_expert(int64_t rows, int experts) {
+  const double per = (double)rows / experts;
+  return per + (experts > 1 ? 1.5 * std::sqrt(per) : 0.0);
+}
+// Where the streaming kernels beat the persistent ones: as long as an expert's rows
+// fit one 192-row tile, with few experts a little further (layer call, persistent /
+// streaming, us: DiT-XL width, 8 experts, 256 tokens 129 / 90, 512 139 / 105, 768
+// 149 / 140, 1024 163 / 169; width 1408, 16 experts, 1024 tokens 252 / 243, 1536
+// 287 / 331; DiT-G width, fp8 weights, 512 tokens 441 / 277, 1024 496 / 388, 2048
+// 643 / 634).
+bool stream_pays(int64_t rows, int experts, bool w8) {
+  return rows_of_full_expert(rows, experts) <= 192.0 || (!w8 && experts <= 8 && rows <= 192ll * experts);
+}
+// Whether 192-row tiles spare an expert a tile over 128-row ones.
+bool stream_tall(int64_t rows, int experts) {
+  const double high = rows_of_full_expert(rows, experts);
+  return std::ceil(high / 192.0) < std::ceil(high / 128.0);
 }
 
 struct Carve {
@@ -38,6 +65,7 @@ struct LayerWorkspace {
   void *h, *slot_out, *shared_h, *shared_out, *modulated;
   int32_t *shared_offsets;
   void *split_ws;    // partial-tile slots of fc2 launches whose last turn is cut along k (16-bit activations)
+  float *slot_part, *shared_part;  // partial rows of a streaming fc2 launch that is cut along k (small batches)
   uint8_t *q_rows;   // (act_quant) fp8 rows of the GEMM about to run: [slots, max(hidden, inter)]
   float *q_scale;    // ... and their scales [slots]
   size_t total;
@@ -55,6 +83,11 @@ bool act_quant_widths_ok(int hidden, int inter) {
 // with fp8 weights (their bf16 shared expert rides alone), no shared expert, or
 // the small batches whose shared fc2 gets a launch of its own.
 bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_rows);
+struct StreamPlan {
+  bool fc1, fc2;                    // the stages that take the streaming kernels
+  int slot_pieces, shared_pieces;   // pieces fc2's k ranges are cut into
+};
+StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, int64_t n_tokens, int64_t max_rows);
 bool layer_may_split_fc2(const dice_moe_layer_t *L, int64_t n_tokens) {
   if (!is_16bit(L->act_dtype) || L->batch_invariant) return false;
   if (L->w_dtype == DICE_FP8_E4M3 || L->shared_inter == 0) return true;
@@ -85,6 +118,14 @@ LayerWorkspace carve_layer(const dice_moe_layer_t *L, int64_t n_tokens, void *ws
   }
   w.modulated = c.take_bytes((size_t)n_tokens * L->hidden * es);  // layer input when the caller's prologue runs here
   w.split_ws = layer_may_split_fc2(L, n_tokens) ? c.take_bytes(persist_split_ws_bytes()) : nullptr;
+  w.slot_part = w.shared_part = nullptr;
+  {
+    // (a skip step has fewer rows, so it may stream where a full step of the same tokens does not)
+    const StreamPlan plan = plan_stream(L, L, n_tokens, n_tokens * (L->top_k > 1 ? L->top_k - 1 : 1));
+    if (plan.fc2 && plan.slot_pieces > 1) w.slot_part = c.take<float>(slots * L->hidden * plan.slot_pieces);
+    if (plan.fc2 && plan.shared_pieces > 1)
+      w.shared_part = c.take<float>((size_t)n_tokens * L->hidden * plan.shared_pieces);
+  }
   w.q_rows = nullptr;
   w.q_scale = nullptr;
   if (L->act_quant) {
@@ -305,6 +346,19 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
       pb1.prob[0].w_scale = w1_scale;
       pb2.prob[0].w_scale = w2_scale;
     }
+    if (!scatter_to_slots && stream_choice() == 0 && stream_pays(max_rows, n_experts, w_dtype == DICE_FP8_E4M3)) {
+      StreamBatch s1{}, s2{};
+      s1.n_problems = s2.n_problems = 1;
+      s1.pieces[0] = s2.pieces[0] = 1;
+      s1.tall = s2.tall = stream_tall(max_rows, n_experts);
+      s1.prob[0] = pb1.prob[0];
+      s2.prob[0] = pb2.prob[0];
+      if (stream_supported(s1, m1) && stream_supported(s2, kFc2)) {
+        rc = stages & 1 ? launch_stream(s1, m1, act_dtype, s) : (int)DICE_OK;
+        if (rc || !(stages & 2)) return rc;
+        return launch_stream(s2, kFc2, act_dtype, s);
+      }
+    }
     const bool few = few_rows_per_group(max_rows, n_experts);
     fc1_persist = gemm_config_allows_persistent(m1) && !(few && gemm_config_is_default(m1)) && persist_supported(pb1, m1);
     fc2_persist = !scatter_to_slots && gemm_config_allows_persistent(kFc2) &&
@@ -418,6 +472,29 @@ bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_r
   const int64_t m_tiles = max_rows / 256 + L->n_experts + n_tokens / 256 + 1;
   const int64_t tiles = m_tiles * ((L->hidden + 255) / 256);
   return tiles * 16 <= (int64_t)persist_cu_count() * (L->shared_inter > L->inter ? 7 : 6);
+}
+
+// Small batches take the streaming kernels (grouped_gemm_stream.hip).  The persistent
+// kernels' 256-row tiles are then mostly padding and their launches a turn or two of
+// which the last is nearly empty.
+// An fc2 launch with few tiles is cut along k into pieces of about 2304 (fp32
+// partial rows, added up by the combine kernel): at DiT-XL width 9 tiles per
+// expert and 72 steps, 39 us in two pieces against 50 whole.  Whether and how far
+// depends on the layer's shape alone, not on the batch, so that a skip step and
+// the full step it belongs to add up their rows alike.
+StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, int64_t n_tokens, int64_t max_rows) {
+  StreamPlan plan{false, false, 1, 1};
+  const int choice = stream_choice();
+  if (!is_16bit(L->act_dtype) || L->act_quant || L->batch_invariant || choice < 0 || !persist_split_allowed()) return plan;
+  if (choice == 0 && !stream_pays(max_rows, L->n_experts, LE->w_dtype == DICE_FP8_E4M3)) return plan;
+  plan.fc1 = plan.fc2 = true;
+  const int n_tiles = (L->hidden + 127) / 128;
+  if ((L->n_experts + (L->shared_inter > 0)) * n_tiles < 160 && (L->top_k == 1 || L->top_k == 2 || L->top_k == 4)) {
+    auto pieces = [](int k) { return k < 3456 ? 1 : k < 5760 ? 2 : k < 8064 ? 3 : 4; };
+    plan.slot_pieces = pieces(L->inter);
+    plan.shared_pieces = pieces(L->shared_inter);
+  }
+  return plan;
 }
 
 int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_layer_t *LE, const void *x,
@@ -578,6 +655,11 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
   // (bf16) gets launches of its own.
   bool done = false;
   const bool w8 = LE->w_dtype == DICE_FP8_E4M3;
+  const void *emit_rows = emit.rows, *shared_rows = w.shared_out;
+  StreamPlan plan = plan_stream(L, LE, n_tokens, max_rows);
+  if (w8 && !(LE->w1_scale && LE->w2_scale)) plan = StreamPlan{false, false, 1, 1};
+  // (rows that a later call combines are kept in the entry, whole)
+  if (put || work_in || emit_in) plan.slot_pieces = 1;
   if (LE->act_quant) {
     // fp8 activations too: the routed experts run on the fp8 matrix pipe, each
     // GEMM behind a quantiser of its input rows; the shared expert (bf16)
@@ -618,7 +700,66 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
     if (rc) return rc;
     stamp(8, s);
     done = true;
-  } else if (is_16bit(L->act_dtype) && (LE->w_dtype == L->act_dtype || (w8 && LE->w1_scale && LE->w2_scale))) {
+  } else if (plan.fc1) {
+    const bool swiglu = L->act_variant == DICE_ACT_SWIGLU;
+    const int m1 = swiglu ? kFc1Swiglu : kFc1Gelu;
+    const int si = L->shared_inter;
+    StreamBatch f1{}, f2{};
+    auto fc1_problem = [&](const void *a, const int32_t *offsets, int experts, const void *wt1, const float *b1, void *h,
+                           int inter, int64_t rows) {
+      return PersistProblem{a, L->hidden, offsets, experts, wt1, swiglu ? 2 * inter : inter, swiglu ? inter : 0,
+                            swiglu ? nullptr : b1, h, inter, inter, L->hidden, (int)rows, nullptr, 1};
+    };
+    auto fc2_problem = [&](const void *a, const int32_t *offsets, int experts, const void *wt2, const float *b2, void *out,
+                           int inter, int64_t rows) {
+      return PersistProblem{a, inter, offsets, experts, wt2, L->hidden, 0, swiglu ? nullptr : b2, out, L->hidden,
+                            L->hidden, inter, (int)rows, nullptr, 1};
+    };
+    f1.prob[0] = fc1_problem(work.x, work.offsets, L->n_experts, LE->w1, LE->b1, w.h, L->inter, max_rows);
+    f1.prob[0].a_rows = work.perm;
+    f1.prob[0].a_div = L->top_k;
+    f1.prob[0].a_src_rows = (int)n_tokens;
+    f2.prob[0] = fc2_problem(w.h, work.offsets, L->n_experts, LE->w2, LE->b2,
+                             plan.slot_pieces > 1 ? (void *)w.slot_part : work.rows, L->inter, max_rows);
+    f1.n_problems = f2.n_problems = 1;
+    f1.pieces[0] = f1.pieces[1] = 1;
+    f2.pieces[0] = plan.slot_pieces;
+    if (w8) {
+      f1.prob[0].w_scale = LE->w1_scale;
+      f2.prob[0].w_scale = LE->w2_scale;
+    }
+    f1.tall = f2.tall = stream_tall(max_rows, L->n_experts);
+    if (si > 0) {
+      f1.prob[f1.n_problems++] = fc1_problem(x, w.shared_offsets, 1, L->shared_w1, L->shared_b1, w.shared_h, si, n_tokens);
+      f2.pieces[1] = plan.shared_pieces;
+      f2.prob[f2.n_problems++] = fc2_problem(w.shared_h, w.shared_offsets, 1, L->shared_w2, L->shared_b2,
+                                             plan.shared_pieces > 1 ? (void *)w.shared_part : w.shared_out, si, n_tokens);
+      // (the longest tiles first; fp8 weights are the first problem's)
+      if (!w8 && si / plan.shared_pieces > L->inter / plan.slot_pieces) {
+        std::swap(f2.prob[0], f2.prob[1]);
+        std::swap(f2.pieces[0], f2.pieces[1]);
+      }
+    }
+    if (stream_supported(f1, m1) && stream_supported(f2, kFc2)) {
+      stamp(3, s);
+      rc = launch_stream(f1, m1, L->act_dtype, s);
+      if (rc) return rc;
+      stamp(4, s);
+      stamp(5, s);
+      stamp(6, s);
+      rc = launch_stream(f2, kFc2, L->act_dtype, s);
+      if (rc) return rc;
+      stamp(7, s);
+      stamp(8, s);
+      done = true;
+      if (plan.slot_pieces > 1) emit_rows = w.slot_part;
+      if (plan.shared_pieces > 1) shared_rows = w.shared_part;
+    } else {
+      plan = StreamPlan{false, false, 1, 1};
+    }
+  }
+  if (!done && !LE->act_quant && is_16bit(L->act_dtype) &&
+      (LE->w_dtype == L->act_dtype || (w8 && LE->w1_scale && LE->w2_scale))) {
     const bool swiglu = L->act_variant == DICE_ACT_SWIGLU;
     const int m1 = swiglu ? kFc1Swiglu : kFc1Gelu;
     PersistBatch f1{}, f2{};
@@ -717,10 +858,10 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
       stamp(stage == 1 ? 5 : 8, s);
     }
   }
-  rc = combine_impl(emit.rows, emit.inv_perm, combine_wt, w.shared_out, mask,
+  rc = combine_impl(emit_rows, emit.inv_perm, combine_wt, shared_rows, mask,
                     combine_mode == 2 ? cache_in : nullptr, combine_mode == 1 ? cache_out : nullptr, y,
                     L->act_dtype, n_tokens, L->top_k, L->hidden, resid, caller ? caller->gate : nullptr,
-                    caller ? caller->tokens_per_sample : 1, stream);
+                    caller ? caller->tokens_per_sample : 1, stream, plan.slot_pieces, max_rows, plan.shared_pieces);
   stamp(kStages, s);
   return rc;
 }
