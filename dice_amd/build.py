@@ -25,6 +25,7 @@ SOURCES = [
     "modulate.hip",
     "quant.hip",
     "grouped_gemm_f32.hip",
+    "grouped_gemm_split.hip",
     "grouped_gemm_bf16.hip",
     "grouped_gemm_f16.hip",
     "grouped_gemm_stream.hip",

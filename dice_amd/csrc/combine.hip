@@ -189,16 +189,14 @@ int launch_combine(const void *slot_out, const int32_t *inv_perm, const float *w
                      (const Pack<T> *)cache_in, (Pack<T> *)cache_out, (Pack<T> *)y, n_tokens, top_k, \
                      vec_per_row, (const Pack<T> *)resid, (const Pack<T> *)gate, tokens_per_sample, slot_pieces, \
                      slot_rows * vec_per_row, shared_pieces)
-  if constexpr (Pack<T>::kN == 8) {
-    if (split) {
-      switch (top_k) {
-        case 1: DICE_COMBINE_LAUNCH(1, true); break;
-        case 2: DICE_COMBINE_LAUNCH(2, true); break;
-        case 4: DICE_COMBINE_LAUNCH(4, true); break;
-        default: return fail(DICE_ERR_UNSUPPORTED, "dice_combine: partial rows with top_k %d", top_k);
-      }
-      return launch_status("dice_combine");
+  if (split) {
+    switch (top_k) {
+      case 1: DICE_COMBINE_LAUNCH(1, true); break;
+      case 2: DICE_COMBINE_LAUNCH(2, true); break;
+      case 4: DICE_COMBINE_LAUNCH(4, true); break;
+      default: return fail(DICE_ERR_UNSUPPORTED, "dice_combine: partial rows with top_k %d", top_k);
     }
+    return launch_status("dice_combine");
   }
   switch (top_k) {
     case 1: DICE_COMBINE_LAUNCH(1); break;

@@ -215,9 +215,13 @@ struct StreamBatch {
   // fc2: pieces a problem's k range is cut into.  With more than one the kernel writes
   // fp32 partial rows: piece i of row r at c + (i * max_rows + r) * ldc floats.
   int pieces[2];
-  bool tall;   // 192-row tiles instead of 128-row ones
+  bool tall;   // 192-row tiles instead of 128-row ones (16-bit activations)
+  const int32_t *c_rows;   // (fp32, one problem) fc2 writes grouped row r to row c_rows[r]
 };
 bool stream_supported(const StreamBatch &b, int mode);
+// fp32 activations and weights as three bf16 parts on the bf16 matrix pipe (grouped_gemm_split.hip).
+bool split_f32_supported(const StreamBatch &b);
+int launch_grouped_gemm_split_f32(const StreamBatch &b, int mode, hipStream_t s);
 int launch_grouped_gemm_stream(const StreamBatch &b, int mode, hipStream_t s);
 int launch_grouped_gemm_stream_f16(const StreamBatch &b, int mode, hipStream_t s);
 
@@ -243,7 +247,7 @@ int ln_modulate_route_impl(const void *x, const void *shift, const void *scale, 
                            const float *gate_bias, int n_experts, int top_k, int norm_topk_prob, int32_t *topk_idx,
                            float *topk_weight, void *stream);
 // slot_pieces / shared_pieces > 1: the rows are fp32 partial rows that add up to a row (piece i of the slot rows
-// lies i * slot_rows rows on, of the shared rows i * n_tokens rows); 16-bit types, top_k 1, 2 or 4.
+// lies i * slot_rows rows on, of the shared rows i * n_tokens rows); top_k 1, 2 or 4.
 int combine_impl(const void *slot_out, const int32_t *inv_perm, const float *topk_weight,
                  const void *shared_out, const uint8_t *skip_mask, const void *cache_in, void *cache_out,
                  void *y, int dtype, int64_t n_tokens, int top_k, int hidden, const void *resid,

@@ -1,0 +1,367 @@
+// fp32 grouped expert GEMMs on the bf16 matrix pipe.
+//
+// The fp32 matrix instructions run at a sixteenth of the bf16 rate.  An fp32 number is
+// the exact sum of three bf16 numbers, each the rounding of what the ones before it
+// leave (8 + 8 + 8 significant bits), so a product of two of them is nine products of
+// bf16 numbers, every one exact in the matrix pipe's fp32 accumulator.  Six are formed,
+// the smallest first:
+//   a3 b1, a2 b2, a1 b3, a2 b1, a1 b2, a1 b1;
+// the three left out are together below 2^-25 of the product, of either sign: less than
+// the rounding of one addition.  (The decomposition is the classical one for products
+// in higher precision from lower-precision parts: T. J. Dekker, Numer. Math. 18, 1971.)
+// Against float64 the rows are as close as those of the fp32 matrix instructions, whose
+// sum is rounded at every second product, here six times in sixteen.  A value that
+// rounds to infinity in bf16 (above 3.39e38) makes the elements it enters NaN.
+//
+// A workgroup multiplies BM grouped rows x BN weight rows.  Rows travel as whole
+// 128-byte lines (32 k) through registers, STAGES lines ahead; a thread holds pairs of
+// 16-byte chunks, the first of which belongs to the line's even sub-step of 16 k and the
+// second to the odd one (both operands alike, so every k meets its partner).  A chunk is
+// split on the way into LDS - three planes of [rows][16] bf16, two buffers - while the
+// matrix pipe multiplies the other buffer: three and a half vector instructions per
+// value against six products of 32 cycles per 32 x 32 x 16 block.  One barrier per
+// sub-step.
+//
+// Bound: large shapes by the matrix pipe under the power limit (256 x 256 tiles: 208
+// TFLOP/s of fp32 products, 1250 of bf16 ones, 14 % faster on zero operands; the fp32
+// instructions reached 116-125), small ones by the chain load - split - LDS - product of
+// a sub-step (about 0.3 us), whatever the tile, the depth of the prefetch or the order
+// of the instructions.  Both stages of DiT-B width (8192 tokens, shared expert
+// included) 2470 -> 1510 us; of DiT-S width, 256 tokens, 105 -> 39 us.
+#include <cmath>
+#include <type_traits>
+
+#include "stream_tiles.h"
+
+namespace dice {
+namespace {
+
+template <int V> using int_c = std::integral_constant<int, V>;
+constexpr uint32_t kRsrc = 0x00020000u;
+constexpr uint32_t kNowhere = 0x80000000u;
+
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+template <int MODE_, int TM_, int TN_, int WM_, int WN_, int STAGES_>
+struct SplitGeom {
+  static constexpr int MODE = MODE_, TM = TM_, TN = TN_, WM = WM_, WN = WN_, STAGES = STAGES_;
+  static constexpr int WAVES = WM * WN, THREADS = WAVES * 64;
+  static constexpr bool SWIGLU = MODE == kFc1Swiglu;
+  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BN_OUT = SWIGLU ? BN / 2 : BN;
+  static constexpr int ROWS = BM + BN, PASS_ROWS = WAVES * 16;   // rows of a load pass (four threads each)
+  static constexpr int A_PASSES = BM / PASS_ROWS, PASSES = ROWS / PASS_ROWS;
+  static_assert(BM % PASS_ROWS == 0 && BN % PASS_ROWS == 0, "whole passes of either operand");
+  static constexpr int PLANE = ROWS * 32, BUFFER = 3 * PLANE;
+  static constexpr size_t LDS = 2 * BUFFER;
+};
+// Byte of 16-byte half `h` (8 k) of `row` in a plane: rows eight apart would meet in the same banks.
+__device__ __forceinline__ int plane_off(int row, int h) { return row * 32 + ((h ^ ((row >> 3) & 1)) << 4); }
+
+// Three bf16 parts of two values each; a + b + c is the value.
+struct Parts {
+  uint32_t a, b, c;
+};
+// v - (half of p that minus_one selects), exact: one instruction instead of an unpack and a subtraction
+// (minus_one is bf16 -1 in one half and 0 in the other).
+__device__ __forceinline__ float less_half(float v, uint32_t p, uint32_t minus_one) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, p), __builtin_bit_cast(bf16x2_t, minus_one), v, false);
+}
+__device__ __forceinline__ Parts split_pair(float x, float y, uint32_t minus_lo, uint32_t minus_hi) {
+  auto round_pair = [](float u, float v) {
+    const bf16x2_t r = {(bf16_t)u, (bf16_t)v};
+    return __builtin_bit_cast(uint32_t, r);
+  };
+  Parts p;
+  p.a = round_pair(x, y);
+  x = less_half(x, p.a, minus_lo);
+  y = less_half(y, p.a, minus_hi);
+  p.b = round_pair(x, y);
+  x = less_half(x, p.b, minus_lo);
+  y = less_half(y, p.b, minus_hi);
+  p.c = round_pair(x, y);
+  return p;
+}
+
+template <typename G>
+__device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *lds) {
+  constexpr int MODE = G::MODE, TM = G::TM, TN = G::TN, WM = G::WM, WN = G::WN, STAGES = G::STAGES;
+  constexpr bool SWIGLU = G::SWIGLU;
+  constexpr int BM = G::BM, BN_OUT = G::BN_OUT, PASSES = G::PASSES, A_PASSES = G::A_PASSES, PASS_ROWS = G::PASS_ROWS;
+  const StreamTile t = locate_stream_tile<BM, BN_OUT, BM, BN_OUT>(b);
+  if (!t.active) return;
+  const PersistProblem &p = b.prob[t.prob];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uniform(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int k = p.k, n = p.n;
+  const int all_lines = k / 32;
+  int line0 = 0, lines = all_lines;
+  if (t.pieces > 1) {
+    line0 = (int)((unsigned)(all_lines * t.piece) / (unsigned)t.pieces);
+    lines = (int)((unsigned)(all_lines * (t.piece + 1)) / (unsigned)t.pieces) - line0;
+  }
+  lines = uniform(lines);
+
+  // ---- global loads: pass i covers tile rows PASS_ROWS i + tid / 4 (activation rows first), chunks 2 (tid % 4) and the next ----
+  const int ld_row = tid >> 2, ld_pair = tid & 3;
+  uint32_t voff[PASSES];
+  {
+    const uint32_t pitch = (uint32_t)p.lda * 4;
+    uint32_t src[A_PASSES];
+#pragma unroll
+    for (int i = 0; i < A_PASSES; ++i) src[i] = (uint32_t)(i * PASS_ROWS + ld_row);
+    if (p.a_rows) {
+      const int32_t *rows = p.a_rows + t.row0;
+      const uint32_t magic = p.a_div == 1 ? 0u : (uint32_t)(0xffffffffu / (uint32_t)p.a_div + 1u);   // slot / a_div = mulhi(slot, magic)
+#pragma unroll
+      for (int i = 0; i < A_PASSES; ++i) src[i] = (uint32_t)rows[(int)src[i] < t.rows ? src[i] : 0];
+#pragma unroll
+      for (int i = 0; i < A_PASSES; ++i) src[i] = magic ? __umulhi(src[i], magic) : src[i];
+    }
+#pragma unroll
+    for (int i = 0; i < A_PASSES; ++i) {
+      const uint32_t off = src[i] * pitch + ld_pair * 32;
+      voff[i] = i * PASS_ROWS + ld_row < t.rows ? off : kNowhere;
+    }
+    const uint32_t wpitch = (uint32_t)k * 4;
+    const int up = SWIGLU ? p.up_offset : 0;
+#pragma unroll
+    for (int i = A_PASSES; i < PASSES; ++i) {
+      const int r = (i - A_PASSES) * PASS_ROWS + ld_row;
+      const int col = t.n0 + (SWIGLU ? (r >> 5) * 16 + (r & 15) : r);   // (strips of 16 gate and the 16 matching up rows)
+      const uint32_t off = (uint32_t)(col + ((r & 16) != 0 ? up : 0)) * wpitch + ld_pair * 32;
+      voff[i] = col < n ? off : kNowhere;
+    }
+  }
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      p.a_rows ? (void *)p.a : (void *)((const float *)p.a + (size_t)t.row0 * p.lda), 0,
+      (uint32_t)(p.a_rows ? p.a_src_rows : t.rows) * (uint32_t)p.lda * 4u, kRsrc);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)((const float *)p.w + (size_t)t.expert * p.w_rows * k), 0, (uint32_t)p.w_rows * (uint32_t)k * 4u, kRsrc);
+  u32x4_t raw[STAGES][PASSES][2];
+  auto load_line = [&](int line, int stage) {
+    const int off = uniform((line0 + (line < lines ? line : lines - 1)) * 128);
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        raw[stage][i][c] = __builtin_amdgcn_raw_buffer_load_b128(i < A_PASSES ? ra : rw, voff[i] + c * 16, off, 0);
+  };
+  uint32_t minus_lo = 0xbf80u, minus_hi = 0xbf800000u;
+  asm("" : "+s"(minus_lo), "+s"(minus_hi));   // (kept in registers: as an inline constant -1.0 would sit in the wrong half)
+  // Chunk c of register stage `stage` into LDS buffer `buf`.
+  unsigned char *const wr = lds + plane_off(ld_row, ld_pair >> 1) + (ld_pair & 1) * 8;   // (PASS_ROWS on: the same half order)
+  auto convert = [&](int stage, int c, int buf) {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const f32x4_t v = __builtin_bit_cast(f32x4_t, raw[stage][i][c]);
+      const Parts lo = split_pair(v[0], v[1], minus_lo, minus_hi), hi = split_pair(v[2], v[3], minus_lo, minus_hi);
+      unsigned char *dst = wr + buf * G::BUFFER + i * PASS_ROWS * 32;
+      *reinterpret_cast<u32x2_any_t *>(dst) = u32x2_t{lo.a, hi.a};
+      *reinterpret_cast<u32x2_any_t *>(dst + G::PLANE) = u32x2_t{lo.b, hi.b};
+      *reinterpret_cast<u32x2_any_t *>(dst + 2 * G::PLANE) = u32x2_t{lo.c, hi.c};
+    }
+  };
+
+  const int frag_row = lane & 31, half = lane >> 5;
+  const unsigned char *const rd_a = lds + plane_off(wm * 32 + frag_row, half);
+  const unsigned char *const rd_w = lds + plane_off(BM + wn * TN * 32 + frag_row, half);
+  const int blocks = (t.rows + 31) >> 5;
+  const int live = uniform((blocks - wm + WM - 1) / WM);   // row blocks of this wave (tile blocks wm, wm + WM, ..) that hold rows
+
+#pragma unroll
+  for (int i = 0; i < STAGES; ++i) load_line(i, i);
+
+  auto run = [&](auto live_c) {
+    constexpr int LIVE = decltype(live_c)::value, LV = LIVE > 0 ? LIVE : 1;
+    f32x16_t acc[LV][TN];
+#pragma unroll
+    for (int i = 0; i < LV; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    auto multiply = [&](int buf) {
+      if constexpr (LIVE > 0) {
+        bf16x8_t wf[3][TN], af[3][LV];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            wf[q][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_any_t *>(rd_w + buf * G::BUFFER + q * G::PLANE + j * 32 * 32));
+#pragma unroll
+          for (int i = 0; i < LIVE; ++i)
+            af[q][i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_any_t *>(rd_a + buf * G::BUFFER + q * G::PLANE + i * WM * 32 * 32));
+        }
+        constexpr int order[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+        for (int o = 0; o < 6; ++o)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int i = 0; i < LIVE; ++i)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[order[o][1]][j], af[order[o][0]][i], acc[i][j], 0, 0, 0);
+      }
+    };
+    auto line = [&](int l, auto stage_c) {
+      constexpr int S = decltype(stage_c)::value;
+      multiply(0);
+      convert(S, 1, 1);
+      block_lds_barrier();
+      load_line(l + STAGES, S);
+      multiply(1);
+      convert((S + 1) % STAGES, 0, 0);   // (behind the last line: of a line loaded again, never multiplied)
+      block_lds_barrier();
+    };
+    convert(0, 0, 0);
+    block_lds_barrier();
+    int l = 0;
+    for (; l + STAGES <= lines; l += STAGES) {
+      line(l, int_c<0>{});
+      if constexpr (STAGES > 1) line(l + 1, int_c<1 % STAGES>{});
+      if constexpr (STAGES > 2) line(l + 2, int_c<2 % STAGES>{});
+      if constexpr (STAGES > 3) line(l + 3, int_c<3 % STAGES>{});
+    }
+    if constexpr (STAGES > 1) {
+      if (l < lines) line(l, int_c<0>{});
+    }
+    if constexpr (STAGES > 2) {
+      if (l + 1 < lines) line(l + 1, int_c<1>{});
+      if (l + 2 < lines) line(l + 2, int_c<2 % STAGES>{});
+    }
+
+    // ---- epilogue: lane holds row frag_row, columns 8 q + 4 half + {0..3} of each block ----
+    if constexpr (LIVE > 0) {
+      constexpr int BW = SWIGLU ? 16 : 32;   // output columns of a weight block
+      const float *bias = p.bias ? p.bias + (size_t)t.expert * n : nullptr;
+      float *const out = (float *)p.c + (size_t)(t.pieces > 1 ? t.piece : 0) * p.max_rows * p.ldc;
+      size_t dst[LV];
+#pragma unroll
+      for (int i = 0; i < LV; ++i) {
+        const int m = (i * WM + wm) * 32 + frag_row;
+        dst[i] = (size_t)(b.c_rows ? b.c_rows[t.row0 + (m < t.rows ? m : 0)] : t.row0 + m) * p.ldc;
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < BW / 8; ++q) {
+          const int col = t.n0 + (wn * TN + j) * BW + half * 4 + q * 8;
+          const int ccol = col < n ? col : 0;
+          f32x4_t sb;
+          if (!SWIGLU) sb = bias && t.piece == 0 ? *reinterpret_cast<const f32x4_t *>(bias + ccol) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < LIVE; ++i) {
+            const int m = (i * WM + wm) * 32 + frag_row;
+            f32x4_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float x = acc[i][j][q * 4 + r];
+              if (SWIGLU) {
+                x = silu_fast(x) * acc[i][j][8 + q * 4 + r];
+              } else {
+                x += sb[r];
+                if (MODE == kFc1Gelu) x = gelu_tanh_fast(x);
+              }
+              v[r] = x;
+            }
+            if (m < t.rows && col < n) *reinterpret_cast<f32x4_t *>(out + dst[i] + col) = v;
+          }
+        }
+    }
+  };
+  if constexpr (TM >= 4) {
+    if (live >= 4) return run(int_c<4>{});
+    if (live >= 3) return run(int_c<3>{});
+  }
+  if constexpr (TM >= 2) {
+    if (live >= 2) return run(int_c<2>{});
+  }
+  if (live >= 1) return run(int_c<1>{});
+  run(int_c<0>{});
+}
+
+template <typename G>
+__global__ __launch_bounds__(G::THREADS, 2) void grouped_gemm_split_kernel(StreamBatch b) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char split_lds[];
+  split_body<G>(b, split_lds);
+}
+
+template <typename G>
+int launch_shape(const StreamBatch &b, hipStream_t s) {
+  const int64_t grid = stream_grid(b, G::BM, G::BN_OUT, G::BM, G::BN_OUT);
+  auto kern = grouped_gemm_split_kernel<G>;
+  static thread_local bool configured = G::LDS <= 64 * 1024;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS);
+    if (e != hipSuccess) return fail(DICE_ERR_LAUNCH, "grouped_gemm_split: LDS attribute: %s", hipGetErrorString(e));
+    configured = true;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(G::THREADS), G::LDS, s, b);
+  return launch_status("grouped_gemm_split");
+}
+
+// Tiles of a launch under a uniform routing (half a partial tile per expert), each over its whole k range.
+double expected_tiles(const StreamBatch &b, int bm, int bn) {
+  double t = 0;
+  for (int i = 0; i < b.n_problems; ++i) {
+    const PersistProblem &p = b.prob[i];
+    const double m = (double)p.max_rows / bm;
+    t += (p.n_experts > 1 ? m + 0.5 * p.n_experts : std::ceil(m)) * ((p.n + bn - 1) / bn);
+  }
+  return t;
+}
+// Which part of its turns' time (one workgroup per compute unit) a launch of `tiles` has work for.
+double filled_turns(double tiles) {
+  const double turns = tiles / persist_cu_count();
+  return turns / std::ceil(turns);
+}
+
+// 64 x 64 tiles while all of them make a few turns (DiT-S width, SwiGLU fc1, 64 x 64 /
+// 128 x 128, us: 1024 tokens, 2100 tiles, 53 / 60; 2048 tokens 97 / 90; DiT-B width, GELU,
+// 1024 tokens, 2100 tiles, 103 / 108; fc2's longer tiles cross earlier: DiT-B width,
+// 1024 tokens, 620 tiles, 115 / 154; 2048 tokens, 1200 tiles, 188 / 178).  The larger
+// ones run one workgroup per compute unit and pay where their last turn is fairly
+// full (DiT-B width, 8192 tokens: fc1 128 x 128 / 256 x 256 1080 / 996; fc2 128 x
+// 128 / 256 x 128, 2.4 turns of three, 580 / 530; 4096 tokens, 1.2 of two, 300 / 339).
+template <int MODE>
+int launch_mode(const StreamBatch &b, hipStream_t s) {
+#ifdef SPLIT_PROBE
+  SPLIT_PROBE
+#endif
+  constexpr int cols = MODE == kFc1Swiglu ? 2 : 1;   // weight rows per output column
+  const double cus = persist_cu_count();
+  if (expected_tiles(b, 64, 64 / cols) <= (MODE == kFc2 ? 4.0 : 9.0) * cus) return launch_shape<SplitGeom<MODE, 1, 1, 2, 2, 2>>(b, s);
+  if (filled_turns(expected_tiles(b, 256, 256 / cols)) >= 0.87) return launch_shape<SplitGeom<MODE, 2, 4, 4, 2, 1>>(b, s);
+  if constexpr (MODE == kFc2) {
+    if (filled_turns(expected_tiles(b, 256, 128)) >= 0.72) return launch_shape<SplitGeom<MODE, 2, 2, 4, 2, 2>>(b, s);
+  }
+  return launch_shape<SplitGeom<MODE, 2, 2, 2, 2, 2>>(b, s);
+}
+
+}  // namespace
+
+bool split_f32_supported(const StreamBatch &b) {
+  int groups = 0;
+  for (int i = 0; i < b.n_problems; ++i) {
+    const PersistProblem &p = b.prob[i];
+    groups += p.n_experts;
+    if (p.k % 32 != 0 || b.pieces[i] < 1 || b.pieces[i] > p.k / 64) return false;
+    if (p.n % 8 != 0 || p.lda % 4 != 0 || p.ldc % 4 != 0) return false;
+    if ((size_t)p.w_rows * p.k * 4 >= (1ull << 31)) return false;
+    const size_t a_rows = p.a_rows ? (size_t)p.a_src_rows : 256;
+    if (a_rows * p.lda * 4 >= (1ull << 31)) return false;
+    if (p.a_rows && (p.a_div < 1 || p.a_div > 16 || (int64_t)p.a_src_rows * p.a_div >= (1ll << 28))) return false;
+  }
+  return groups >= 1 && groups <= kWave;
+}
+
+int launch_grouped_gemm_split_f32(const StreamBatch &b, int mode, hipStream_t s) {
+  switch (mode) {
+    case kFc1Swiglu: return launch_mode<kFc1Swiglu>(b, s);
+    case kFc1Gelu: return launch_mode<kFc1Gelu>(b, s);
+    default: return launch_mode<kFc2>(b, s);
+  }
+}
+
+}  // namespace dice

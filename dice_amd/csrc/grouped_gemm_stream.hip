@@ -31,7 +31,7 @@
 // Compiled for bf16 and, through grouped_gemm_stream_f16.hip, for fp16.
 #include <type_traits>
 
-#include "gemm_common.h"
+#include "stream_tiles.h"
 
 #ifndef DICE_STREAM_F16
 #define DICE_STREAM_F16 0
@@ -79,69 +79,6 @@ __device__ __forceinline__ void copy_to_lds(u32x4_t rs, uint32_t dst, uint32_t v
 // At most N of this wave's copies are still in flight, and its LDS reads are done.
 template <int N> __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-
-// What a workgroup multiplies.
-struct StreamTile {
-  int prob, expert, row0, rows, n0, piece, pieces;
-  bool active;
-};
-
-// Tile order: XCD x (= blockIdx % 8) takes an eighth of every problem's tiles; within
-// an expert the m-tile runs fastest, then the piece of k, then the n-tile, so the
-// workgroups that share an L2 and run side by side share weights, then activations.
-template <int BM0, int BN0, int BM1, int BN1>
-__device__ __forceinline__ StreamTile locate(const StreamBatch &b) {
-  const int lane = threadIdx.x & 63;
-  int g_prob = 0, g_expert = 0, begin = 0, cnt = 0, nt = 1, groups = 0, bm = BM0;
-  for (int pi = 0; pi < b.n_problems; ++pi) {
-    const PersistProblem &p = b.prob[pi];
-    const int local = lane - groups;
-    if (local >= 0 && local < p.n_experts) {
-      g_prob = pi;
-      g_expert = local;
-      begin = p.offsets[local];
-      cnt = p.offsets[local + 1] - begin;
-      nt = (pi == 0 ? (p.n + BN0 - 1) / BN0 : (p.n + BN1 - 1) / BN1) * b.pieces[pi];
-      bm = pi == 0 ? BM0 : BM1;
-    }
-    groups += p.n_experts;
-  }
-  const int mt = (int)((unsigned)(cnt + bm - 1) / (unsigned)bm), tiles = mt * nt;
-  int inc = tiles;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const int up = __shfl_up(inc, o, kWave);
-    if (lane >= o) inc += up;
-  }
-  const int xcd = blockIdx.x % kNumXcd;
-  int j = blockIdx.x / kNumXcd, id = -1, first_group = 0;
-  for (int pi = 0; pi < b.n_problems; ++pi) {
-    const int last = first_group + b.prob[pi].n_experts - 1;
-    const int base = __builtin_amdgcn_readlane(inc - tiles, first_group);
-    const int total = __builtin_amdgcn_readlane(inc, last) - base;
-    const int lo = (int)((unsigned)(total * xcd) / kNumXcd), hi = (int)((unsigned)(total * (xcd + 1)) / kNumXcd);
-    if (id < 0 && j < hi - lo) id = base + lo + j;
-    j -= hi - lo;
-    first_group = last + 1;
-  }
-  StreamTile t;
-  t.active = id >= 0;
-  if (!t.active) return t;
-  const int g = __builtin_ctzll(__ballot(id >= inc - tiles && id < inc));
-  const int r = id - __builtin_amdgcn_readlane(inc - tiles, g);
-  const int g_mt = __builtin_amdgcn_readlane(mt, g), g_cnt = __builtin_amdgcn_readlane(cnt, g);
-  const int q = (int)((unsigned)r / (unsigned)g_mt), m = r - q * g_mt;
-  t.prob = __builtin_amdgcn_readlane(g_prob, g);
-  t.expert = __builtin_amdgcn_readlane(g_expert, g);
-  const int g_bm = BM0 == BM1 ? BM0 : t.prob == 0 ? BM0 : BM1, g_bn = BN0 == BN1 ? BN0 : t.prob == 0 ? BN0 : BN1;
-  t.row0 = __builtin_amdgcn_readlane(begin, g) + m * g_bm;
-  t.rows = uniform(g_cnt - m * g_bm < g_bm ? g_cnt - m * g_bm : g_bm);
-  t.pieces = b.pieces[t.prob];
-  const int nq = t.pieces == 1 ? q : (int)((unsigned)q / (unsigned)t.pieces);
-  t.piece = uniform(q - nq * t.pieces);
-  t.n0 = uniform(nq * g_bn);
-  return t;
 }
 
 // TM x TN blocks of 32 x 32 per wave, WM x WN waves; KB: bytes of a weight row per
@@ -455,7 +392,7 @@ __global__ __launch_bounds__(S0::WM *S0::WN *kWave, 2) void grouped_gemm_stream_
   extern __shared__ __attribute__((aligned(1024))) unsigned char stream_lds[];
   using G0 = StreamGeom<MODE, S0>;
   using G1 = StreamGeom<MODE, S1>;
-  const StreamTile t = locate<G0::BM, G0::BN_OUT, G1::BM, G1::BN_OUT>(b);
+  const StreamTile t = locate_stream_tile<G0::BM, G0::BN_OUT, G1::BM, G1::BN_OUT>(b);
   if (!t.active) return;
   if constexpr (std::is_same_v<S0, S1>) {
     stream_body<MODE, S0>(b, t, stream_lds);
@@ -479,14 +416,8 @@ int launch_shape(const StreamBatch &b, hipStream_t s) {
     if (e != hipSuccess) return fail(DICE_ERR_LAUNCH, "streaming expert GEMM: LDS attribute: %s", hipGetErrorString(e));
     configured = true;
   }
-  int64_t per_xcd = 0;
-  for (int i = 0; i < b.n_problems; ++i) {
-    const PersistProblem &p = b.prob[i];
-    const int bm = i == 0 ? G0::BM : G1::BM, bn = i == 0 ? G0::BN_OUT : G1::BN_OUT;
-    const int64_t m_tiles = p.n_experts == 1 ? ((int64_t)p.max_rows + bm - 1) / bm : (int64_t)p.max_rows / bm + p.n_experts;
-    per_xcd += (m_tiles * ((p.n + bn - 1) / bn) * b.pieces[i] + kNumXcd - 1) / kNumXcd;
-  }
-  hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * kNumXcd)), dim3(G0::WAVES * kWave), lds, s, b);
+  const int64_t grid = stream_grid(b, G0::BM, G0::BN_OUT, G1::BM, G1::BN_OUT);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(G0::WAVES * kWave), lds, s, b);
   return launch_status("grouped_gemm_stream");
 }
 

@@ -22,6 +22,7 @@ int launch_persist(const PersistBatch &b, int mode, int act_dtype, hipStream_t s
 }
 
 int launch_stream(const StreamBatch &b, int mode, int act_dtype, hipStream_t s) {
+  if (act_dtype == DICE_F32) return launch_grouped_gemm_split_f32(b, mode, s);
   return act_dtype == DICE_F16 ? launch_grouped_gemm_stream_f16(b, mode, s) : launch_grouped_gemm_stream(b, mode, s);
 }
 
@@ -319,46 +320,52 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
   hipStream_t s = (hipStream_t)stream;
   const bool swiglu = act_variant == DICE_ACT_SWIGLU;
 
-  // 16-bit activations: each stage takes the persistent kernel where it applies
+  // fp32 takes the split kernels, few rows with 16-bit activations the streaming ones.  Otherwise,
+  // with 16-bit activations, each stage takes the persistent kernel where it applies
   // (fc1 addresses rows through the permutation itself in its SwiGLU form; fc2
   // writes grouped rows, so a scatter to slot order stays with the
   // permutation-addressed kernel), unless the tuning hook names a tiling.
   const int m1 = swiglu ? kFc1Swiglu : kFc1Gelu;
   PersistBatch pb1{}, pb2{};
   bool fc1_persist = false, fc2_persist = false;
+  pb1.n_problems = pb2.n_problems = 1;
+  pb1.prob[0] = PersistProblem{x, hidden, offsets, n_experts, w1, swiglu ? 2 * inter : inter, inter,
+                               swiglu ? nullptr : b1, h, inter, inter, hidden, (int)max_rows};
+  if (perm) {
+    // This entry point is not told how many rows x has: the row addresses get
+    // the widest range the kernel can address (the permutation-addressed
+    // kernel checks none either); slots beyond it fall back to that kernel.
+    pb1.prob[0].a_rows = perm;
+    pb1.prob[0].a_div = slots_per_token;
+    const int64_t by_slots = ((1ll << 28) - 1) / slots_per_token;
+    const int64_t by_bytes = ((1ll << 31) - 1) / ((int64_t)hidden * dtype_size(act_dtype));
+    pb1.prob[0].a_src_rows = (int)(by_slots < by_bytes ? by_slots : by_bytes);
+  }
+  pb2.prob[0] = PersistProblem{h, inter, offsets, n_experts, w2, hidden, 0, swiglu ? nullptr : b2,
+                               out, hidden, hidden, inter, (int)max_rows};
+  if (w_dtype == DICE_FP8_E4M3) {
+    pb1.prob[0].w_scale = w1_scale;
+    pb2.prob[0].w_scale = w2_scale;
+  }
+  StreamBatch s1{}, s2{};
+  s1.n_problems = s2.n_problems = 1;
+  s1.pieces[0] = s2.pieces[0] = 1;
+  s1.prob[0] = pb1.prob[0];
+  s2.prob[0] = pb2.prob[0];
+  bool streams = false;
+  if (act_dtype == DICE_F32) {
+    if (scatter_to_slots) s2.c_rows = perm;
+    streams = gemm_config_is_default(m1) && gemm_config_is_default(kFc2) && split_f32_supported(s1) && split_f32_supported(s2);
+  } else if (!scatter_to_slots && stream_choice() == 0 && stream_pays(max_rows, n_experts, w_dtype == DICE_FP8_E4M3)) {
+    s1.tall = s2.tall = stream_tall(max_rows, n_experts);
+    streams = stream_supported(s1, m1) && stream_supported(s2, kFc2);
+  }
+  if (streams) {
+    rc = stages & 1 ? launch_stream(s1, m1, act_dtype, s) : (int)DICE_OK;
+    if (rc || !(stages & 2)) return rc;
+    return launch_stream(s2, kFc2, act_dtype, s);
+  }
   if (is_16bit(act_dtype)) {
-    pb1.n_problems = pb2.n_problems = 1;
-    pb1.prob[0] = PersistProblem{x, hidden, offsets, n_experts, w1, swiglu ? 2 * inter : inter, inter,
-                                 swiglu ? nullptr : b1, h, inter, inter, hidden, (int)max_rows};
-    if (perm) {
-      // This entry point is not told how many rows x has: the row addresses get
-      // the widest range the kernel can address (the permutation-addressed
-      // kernel checks none either); slots beyond it fall back to that kernel.
-      pb1.prob[0].a_rows = perm;
-      pb1.prob[0].a_div = slots_per_token;
-      const int64_t by_slots = ((1ll << 28) - 1) / slots_per_token;
-      const int64_t by_bytes = ((1ll << 31) - 1) / ((int64_t)hidden * 2);
-      pb1.prob[0].a_src_rows = (int)(by_slots < by_bytes ? by_slots : by_bytes);
-    }
-    pb2.prob[0] = PersistProblem{h, inter, offsets, n_experts, w2, hidden, 0, swiglu ? nullptr : b2,
-                                 out, hidden, hidden, inter, (int)max_rows};
-    if (w_dtype == DICE_FP8_E4M3) {
-      pb1.prob[0].w_scale = w1_scale;
-      pb2.prob[0].w_scale = w2_scale;
-    }
-    if (!scatter_to_slots && stream_choice() == 0 && stream_pays(max_rows, n_experts, w_dtype == DICE_FP8_E4M3)) {
-      StreamBatch s1{}, s2{};
-      s1.n_problems = s2.n_problems = 1;
-      s1.pieces[0] = s2.pieces[0] = 1;
-      s1.tall = s2.tall = stream_tall(max_rows, n_experts);
-      s1.prob[0] = pb1.prob[0];
-      s2.prob[0] = pb2.prob[0];
-      if (stream_supported(s1, m1) && stream_supported(s2, kFc2)) {
-        rc = stages & 1 ? launch_stream(s1, m1, act_dtype, s) : (int)DICE_OK;
-        if (rc || !(stages & 2)) return rc;
-        return launch_stream(s2, kFc2, act_dtype, s);
-      }
-    }
     const bool few = few_rows_per_group(max_rows, n_experts);
     fc1_persist = gemm_config_allows_persistent(m1) && !(few && gemm_config_is_default(m1)) && persist_supported(pb1, m1);
     fc2_persist = !scatter_to_slots && gemm_config_allows_persistent(kFc2) &&
@@ -484,6 +491,23 @@ bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_r
 // the full step it belongs to add up their rows alike.
 StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, int64_t n_tokens, int64_t max_rows) {
   StreamPlan plan{false, false, 1, 1};
+  if (L->act_dtype == DICE_F32) {
+    if (!gemm_config_is_default(kFc1Swiglu) || !gemm_config_is_default(kFc2)) return plan;
+    // fp32 always takes the split kernels; an fc2 launch with few tiles (of 64 x 64) is cut into
+    // pieces of about 512 (DiT-S width, 256 tokens, whole / three pieces: 35 / 17 us; 2048 tokens,
+    // 600 tiles, 54 / 50; DiT-B width, 1024 tokens, 620 tiles, whole / four 115 / 105; 2048 tokens,
+    // 1200 tiles, 178 / 170, what the combine kernel's longer reads take back).  By the token
+    // count, which a skip step and its full step share.
+    plan.fc1 = plan.fc2 = true;
+    const int64_t m_tiles = n_tokens * L->top_k / 64 + L->n_experts / 2 + (L->shared_inter > 0 ? (n_tokens + 63) / 64 : 0);
+    if (!L->batch_invariant && persist_split_allowed() && m_tiles * (L->hidden / 64) <= 700 &&
+        (L->top_k == 1 || L->top_k == 2 || L->top_k == 4)) {
+      auto pieces = [](int k) { return k < 640 ? 1 : k < 1664 ? (k + 384) / 512 : 4; };
+      plan.slot_pieces = pieces(L->inter);
+      plan.shared_pieces = L->shared_inter > 0 ? pieces(L->shared_inter) : 1;
+    }
+    return plan;
+  }
   const int choice = stream_choice();
   if (!is_16bit(L->act_dtype) || L->act_quant || L->batch_invariant || choice < 0 || !persist_split_allowed()) return plan;
   if (choice == 0 && !stream_pays(max_rows, L->n_experts, LE->w_dtype == DICE_FP8_E4M3)) return plan;
@@ -740,7 +764,8 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
         std::swap(f2.pieces[0], f2.pieces[1]);
       }
     }
-    if (stream_supported(f1, m1) && stream_supported(f2, kFc2)) {
+    const bool f32 = L->act_dtype == DICE_F32;
+    if (f32 ? split_f32_supported(f1) && split_f32_supported(f2) : stream_supported(f1, m1) && stream_supported(f2, kFc2)) {
       stamp(3, s);
       rc = launch_stream(f1, m1, L->act_dtype, s);
       if (rc) return rc;
@@ -838,7 +863,7 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
     }
   }
   if (!done) {
-    // Every other case (fp32, shapes the persistent kernels do not take): the
+    // Every other case (shapes the kernels above do not take): the
     // per-stage kernels, one launch per stage and expert set, each in its own
     // timer stage.
     const bool shared = L->shared_inter > 0;
