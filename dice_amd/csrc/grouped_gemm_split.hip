@@ -326,9 +326,6 @@ double filled_turns(double tiles) {
 // 128 / 256 x 128, 2.4 turns of three, 580 / 530; 4096 tokens, 1.2 of two, 300 / 339).
 template <int MODE>
 int launch_mode(const StreamBatch &b, hipStream_t s) {
-#ifdef SPLIT_PROBE
-  SPLIT_PROBE
-#endif
   constexpr int cols = MODE == kFc1Swiglu ? 2 : 1;   // weight rows per output column
   const double cus = persist_cu_count();
   if (expected_tiles(b, 64, 64 / cols) <= (MODE == kFc2 ? 4.0 : 9.0) * cus) return launch_shape<SplitGeom<MODE, 1, 1, 2, 2, 2>>(b, s);

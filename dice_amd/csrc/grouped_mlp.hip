@@ -684,6 +684,10 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
   if (w8 && !(LE->w1_scale && LE->w2_scale)) plan = StreamPlan{false, false, 1, 1};
   // (rows that a later call combines are kept in the entry, whole)
   if (put || work_in || emit_in) plan.slot_pieces = 1;
+  // (the workspace was laid out for this layer's own experts and batch: another layer's weight type or an entry's
+  // row count may stream where these do not, and then there are no partial rows to write)
+  if (!w.slot_part) plan.slot_pieces = 1;
+  if (!w.shared_part) plan.shared_pieces = 1;
   if (LE->act_quant) {
     // fp8 activations too: the routed experts run on the fp8 matrix pipe, each
     // GEMM behind a quantiser of its input rows; the shared expert (bf16)

@@ -109,3 +109,41 @@ def test_put_and_skip_on_partial_rows(dev):
     put = blk.run(x, lib.MODE_PUT, mask, None, cache).clone()
     assert torch.equal(put, blk.run(x))
     assert torch.equal(put, blk.run(x, lib.MODE_SKIP, mask, cache, None))
+
+
+def test_entry_with_few_rows_in_a_large_batch(dev):
+    """A lagged call whose entry holds few rows streams where its batch does not: the
+    workspace, laid out for the batch, has no partial rows, so fc2 stays whole."""
+    import ctypes
+    from dice_amd import diep, lib
+    D, E, N, R = 1152, 8, 3000, 64
+    p = _params(D, E, 2, 4, "gelu_tanh", torch.bfloat16, 8)
+    blk = block_from_params(p, D, "gelu_tanh", torch.bfloat16, dev)
+    x = torch.randn(N, D, generator=torch.Generator().manual_seed(9)).bfloat16().to(dev)
+    desc = blk._ensure(x)
+    work = diep.LagEntry(x, E, 2, False, owner=blk)
+    work.ensure_rows()
+    work.x.copy_(x)
+    work.offsets.copy_(torch.arange(E + 1, dtype=torch.int32) * (R // E))
+    work.perm.zero_()
+    work.perm[:R] = torch.arange(R, dtype=torch.int32, device=dev) * 2     # slot 0 of the first R tokens
+    work.inv_perm.fill_(-1)
+    work.inv_perm.view(-1, 2)[:R, 0] = torch.arange(R, dtype=torch.int32, device=dev)
+    work.topk_weight.fill_(0.5)
+    wd = work.desc()
+    wd.max_rows = R
+
+    def call():
+        new = diep.LagEntry(x, E, 2, False, owner=blk)
+        nd, y = new.desc(), torch.empty_like(x)
+        ws = blk._workspace(desc, N, dev)
+        lib.check(lib.load().dice_moe_forward_lagged(
+            ctypes.byref(desc), ctypes.byref(desc), lib.ptr(x), N, 0, None, ctypes.byref(nd), ctypes.byref(wd), None,
+            lib.MODE_PLAIN, None, None, 0, None, lib.ptr(y), None, None, lib.ptr(ws), ws.numel(), lib.stream_ptr()))
+        return y
+
+    y = call()
+    with hook(56):
+        want = call()
+    # (sums of h and y in one order and bf16 roundings of 2^-9 each where a cut turn orders them otherwise)
+    check_rows(y.cpu(), want.cpu(), 8e-3, "streaming vs persistent")
