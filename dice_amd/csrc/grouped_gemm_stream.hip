@@ -447,9 +447,13 @@ bool stream_supported(const StreamBatch &b, int mode) {
 // Tile shapes, eight waves each.  fc1: two workgroups per compute unit; 16-bit weights
 // 128 or 192 rows x 128 weight rows (64 and 80 KB of LDS), fp8 weights (half the bytes
 // per product) 128 x 256 with 64-byte steps (80 KB).  fc2, whose tiles are fewer and
-// longer: one workgroup per compute unit with deeper rings (DiT-XL width, 512 tokens:
-// 36.0 us against 39.9 with the fc1 rings; DiT-G width with fp8 weights 71.5 against
-// 78.8).  The 192-row tile where it saves an expert a second tile, whose workgroup
+// longer: one workgroup per compute unit with deeper rings while all tiles are one
+// turn (layer call, deep / shallow rings, us: DiT-XL width 512 tokens 104 / 106,
+// width 1408, 16 experts, 1200 tokens 261 / 269); with more tiles two workgroups per
+// compute unit, so that the tiles past the first turn start at once instead of
+// behind it (DiT-XL width, 700 tokens 135 / 126, GELU 750 tokens 129 / 120; DiT-G
+// width with fp8 weights, 512 tokens 278 / 267).
+// The 192-row tile where it saves an expert a second tile, whose workgroup
 // would read all of the weights again (fc1 54 us against 61).  Four waves per
 // workgroup, larger tiles with one workgroup per compute unit (fc1) and 64-byte
 // steps of 16-bit weights measured slower: what limits a step is how much
@@ -461,6 +465,7 @@ int DICE_STREAM_LAUNCH(const StreamBatch &b, int mode, hipStream_t s) {
   using Fc2 = Shape<false, 128, 2, 1, 2, 4, 3, 5>;
   using Fc2Tall = Shape<false, 128, 3, 1, 2, 4, 3, 4>;
   using Fc2W8 = Shape<true, 128, 2, 1, 2, 4, 3, 4>;
+  using Fc2W8Pair = Shape<true, 64, 2, 1, 2, 4, 3, 4>;   // (two per compute unit)
   const bool w8 = b.prob[0].w_scale != nullptr;
   switch (mode) {
     case kFc1Swiglu:
@@ -470,6 +475,9 @@ int DICE_STREAM_LAUNCH(const StreamBatch &b, int mode, hipStream_t s) {
       return w8 ? launch_shape<kFc1Gelu, Fc1W8, Fc1Tall>(b, s)
                 : b.tall ? launch_shape<kFc1Gelu, Fc1Tall>(b, s) : launch_shape<kFc1Gelu, Fc1>(b, s);
     default:
+      if (expected_stream_tiles(b, b.tall && !w8 ? 192 : 128, w8 || b.tall ? 192 : 128, 128) > persist_cu_count())
+        return w8 ? launch_shape<kFc2, Fc2W8Pair, Fc1Tall>(b, s)
+                  : b.tall ? launch_shape<kFc2, Fc1Tall>(b, s) : launch_shape<kFc2, Fc1>(b, s);
       return w8 ? launch_shape<kFc2, Fc2W8, Fc2Tall>(b, s)
                 : b.tall ? launch_shape<kFc2, Fc2Tall>(b, s) : launch_shape<kFc2, Fc2>(b, s);
   }

@@ -2,7 +2,7 @@
 #include <cmath>
 #include <utility>
 
-#include "gemm_common.h"
+#include "stream_tiles.h"
 
 namespace dice {
 namespace {
@@ -26,19 +26,24 @@ int launch_stream(const StreamBatch &b, int mode, int act_dtype, hipStream_t s) 
   return act_dtype == DICE_F16 ? launch_grouped_gemm_stream_f16(b, mode, s) : launch_grouped_gemm_stream(b, mode, s);
 }
 
-// Rows of the fuller experts under a uniform routing (1.5 standard deviations).
-double rows_of_full_expert(int64_t rows, int experts) {
-  const double per = (double)rows / experts;
-  return per + (experts > 1 ? 1.5 * std::sqrt(per) : 0.0);
-}
 // Where the streaming kernels beat the persistent ones: as long as an expert's rows
 // fit one 192-row tile, with few experts a little further (layer call, persistent /
-// streaming, us: DiT-XL width, 8 experts, 256 tokens 129 / 90, 512 139 / 105, 768
-// 149 / 140, 1024 163 / 169; width 1408, 16 experts, 1024 tokens 252 / 243, 1536
-// 287 / 331; DiT-G width, fp8 weights, 512 tokens 441 / 277, 1024 496 / 388, 2048
-// 643 / 634).
-bool stream_pays(int64_t rows, int experts, bool w8) {
-  return rows_of_full_expert(rows, experts) <= 192.0 || (!w8 && experts <= 8 && rows <= 192ll * experts);
+// streaming, us: DiT-XL width, 8 experts, 256 tokens 129 / 80, 512 138 / 100; width
+// 1408, 16 experts, 1280 tokens 282 / 274, 1360 282 / 293).  A layer call with a shared
+// expert streams further: the persistent kernels' 256-row tiles then make a turn or two
+// that one expert's few rows or the shared expert's long fc2 tiles decide.  Rows per
+// expert where the two cross (persistent / streaming, us, next to it):
+//   up to 4 experts past 400 (DiT-XL width, 800 tokens, 138 / 130);
+//   up to 8 experts about 290 (SwiGLU, held at 240: 900 tokens 165 / 147, 1100 174 / 165,
+//   1200 167 / 171; GELU 1152 tokens 224 / 166, 1300 202 / 212);
+//   more, GELU: about 185 (1152 wide 239 / 241 at 187; 1408 wide 390 / 384 at 225);
+//   fp8 weights, whose shared expert has launches of its own there: SwiGLU past 288 (DiT-G
+//   width, 2200 tokens 817 / 704), GELU 210 (1600 tokens 608 / 595, 1800 617 / 627).
+bool stream_pays(int64_t rows, int experts, bool w8, bool gelu, bool shared) {
+  if (rows_of_full_expert(rows, experts) <= 192.0) return true;
+  if (!shared) return !w8 && experts <= 8 && rows <= 192ll * experts;
+  const int64_t most = w8 ? (gelu ? 200 : 288) : experts <= 4 ? 384 : experts <= 8 ? (gelu ? 272 : 240) : gelu ? 184 : 0;
+  return rows <= most * experts;
 }
 // Whether 192-row tiles spare an expert a tile over 128-row ones.
 bool stream_tall(int64_t rows, int experts) {
@@ -356,7 +361,7 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
   if (act_dtype == DICE_F32) {
     if (scatter_to_slots) s2.c_rows = perm;
     streams = gemm_config_is_default(m1) && gemm_config_is_default(kFc2) && split_f32_supported(s1) && split_f32_supported(s2);
-  } else if (!scatter_to_slots && stream_choice() == 0 && stream_pays(max_rows, n_experts, w_dtype == DICE_FP8_E4M3)) {
+  } else if (!scatter_to_slots && stream_choice() == 0 && stream_pays(max_rows, n_experts, w_dtype == DICE_FP8_E4M3, !swiglu, false)) {
     s1.tall = s2.tall = stream_tall(max_rows, n_experts);
     streams = stream_supported(s1, m1) && stream_supported(s2, kFc2);
   }
@@ -484,11 +489,15 @@ bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_r
 // Small batches take the streaming kernels (grouped_gemm_stream.hip).  The persistent
 // kernels' 256-row tiles are then mostly padding and their launches a turn or two of
 // which the last is nearly empty.
-// An fc2 launch with few tiles is cut along k into pieces of about 2304 (fp32
+// An fc2 problem with few tiles is cut along k into pieces of about 2304 (fp32
 // partial rows, added up by the combine kernel): at DiT-XL width 9 tiles per
-// expert and 72 steps, 39 us in two pieces against 50 whole.  Whether and how far
-// depends on the layer's shape alone, not on the batch, so that a skip step and
-// the full step it belongs to add up their rows alike.
+// expert and 72 steps, 39 us in two pieces against 50 whole.  The shared expert's
+// tiles are always few, and as long as the launch's longest where its k is: whole
+// beside uncut routed tiles they were its last turn (layer call, shared fc2 whole
+// / cut, us: DiT-G width, fp8 weights, 512 tokens, SwiGLU (k = 4096) 268 / 257, GELU
+// (k = 16384) 371 / 254; width 1408, 16 experts, GELU, 800 tokens 245 / 217).
+// Whether and how far depends on the layer's shape alone, not on the batch, so
+// that a skip step and the full step it belongs to add up their rows alike.
 StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, int64_t n_tokens, int64_t max_rows) {
   StreamPlan plan{false, false, 1, 1};
   if (L->act_dtype == DICE_F32) {
@@ -510,12 +519,13 @@ StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, in
   }
   const int choice = stream_choice();
   if (!is_16bit(L->act_dtype) || L->act_quant || L->batch_invariant || choice < 0 || !persist_split_allowed()) return plan;
-  if (choice == 0 && !stream_pays(max_rows, L->n_experts, LE->w_dtype == DICE_FP8_E4M3)) return plan;
+  if (choice == 0 && !stream_pays(max_rows, L->n_experts, LE->w_dtype == DICE_FP8_E4M3,
+                                  L->act_variant != DICE_ACT_SWIGLU, L->shared_inter > 0)) return plan;
   plan.fc1 = plan.fc2 = true;
   const int n_tiles = (L->hidden + 127) / 128;
-  if ((L->n_experts + (L->shared_inter > 0)) * n_tiles < 160 && (L->top_k == 1 || L->top_k == 2 || L->top_k == 4)) {
+  if (L->top_k == 1 || L->top_k == 2 || L->top_k == 4) {
     auto pieces = [](int k) { return k < 3456 ? 1 : k < 5760 ? 2 : k < 8064 ? 3 : 4; };
-    plan.slot_pieces = pieces(L->inter);
+    if ((L->n_experts + (L->shared_inter > 0)) * n_tiles < 160) plan.slot_pieces = pieces(L->inter);
     plan.shared_pieces = pieces(L->shared_inter);
   }
   return plan;

@@ -1,6 +1,8 @@
 // Tile order of the kernels that take one workgroup per tile and up to two problems
 // per launch (grouped_gemm_stream.hip, grouped_gemm_split.hip).
 #pragma once
+#include <cmath>
+
 #include "gemm_common.h"
 
 namespace dice {
@@ -67,6 +69,23 @@ __device__ __forceinline__ StreamTile locate_stream_tile(const StreamBatch &b) {
   t.piece = __builtin_amdgcn_readfirstlane(q - nq * t.pieces);
   t.n0 = __builtin_amdgcn_readfirstlane(nq * g_bn);
   return t;
+}
+
+// Rows of the fuller experts under a uniform routing (1.5 standard deviations).
+inline double rows_of_full_expert(int64_t rows, int experts) {
+  const double per = (double)rows / experts;
+  return per + (experts > 1 ? 1.5 * std::sqrt(per) : 0.0);
+}
+// Tiles of a launch where every expert is a fuller one: at most as many as compute
+// units are one turn of one workgroup each.
+inline int64_t expected_stream_tiles(const StreamBatch &b, int bm0, int bm1, int bn) {
+  int64_t tiles = 0;
+  for (int i = 0; i < b.n_problems; ++i) {
+    const PersistProblem &p = b.prob[i];
+    const int64_t m_tiles = p.n_experts * (int64_t)std::ceil(rows_of_full_expert(p.max_rows, p.n_experts) / (i == 0 ? bm0 : bm1));
+    tiles += m_tiles * ((p.n + bn - 1) / bn) * b.pieces[i];
+  }
+  return tiles;
 }
 
 // Workgroups of a launch: an upper bound (row counts live on the device; surplus workgroups exit at once).

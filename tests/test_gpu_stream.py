@@ -58,6 +58,9 @@ def _params(D, E, k, ratio, variant, dtype, seed, skew=None):
     (100, 1152, 8, 4, 4, "swiglu", torch.bfloat16),       # the combine of four slots' partial rows
     (90, 1024, 4, 3, 4, "swiglu", torch.bfloat16),        # top-3: fc2 stays whole
     (257, 768, 33, 2, 4, "swiglu", torch.float16),        # many experts, some without rows
+    (200, 1152, 17, 2, 4, "gelu_tanh", torch.bfloat16),   # fc2: routed tiles whole, the shared expert's cut
+    (700, 1152, 8, 2, 4, "swiglu", torch.bfloat16),       # more fc2 tiles than compute units, 192-row tiles
+    (40, 1152, 40, 2, 2, "swiglu", torch.float16),        # ... 128-row tiles, none cut
 ])
 def test_block_on_the_streaming_kernels(dev, N, D, E, k, ratio, variant, dtype):
     skew = None if E < 8 else torch.linspace(2.0, -2.0, E)
@@ -79,6 +82,8 @@ def test_block_on_the_streaming_kernels(dev, N, D, E, k, ratio, variant, dtype):
     (40, 512, 4, 2, "swiglu"),        # 8 k steps of 64 and of 128 (fc2)
     (129, 1024, 4, 2, "gelu_tanh"),   # a second row tile; biases
     (300, 1152, 8, 4, "swiglu"),      # fc2 in two pieces
+    (60, 1024, 20, 4, "gelu_tanh"),   # routed fc2 whole, the shared expert's cut
+    (1500, 1024, 20, 4, "gelu_tanh"), # ... with more tiles than compute units
 ])
 def test_fp8_weights_on_the_streaming_kernels(dev, N, D, E, ratio, variant):
     p = _params(D, E, 2, ratio, variant, torch.bfloat16, N)
