@@ -1,5 +1,5 @@
 // Grouped expert GEMMs for small batches, where a launch is the streaming of its
-// weights: an expert has few rows (up to about 190), every weight is multiplied with
+// weights: an expert has few rows (up to about 190, in layer calls somewhat more), every weight is multiplied with
 // them once, and what counts is that weight bytes are in flight on every compute
 // unit from the first microsecond to the last.  Bound: HBM (this card streams 6.1
 // TB/s whatever the order of the rows, as long as whole 128-byte lines are asked for
@@ -23,7 +23,7 @@
 // Measured, layer call, against the persistent kernels: DiT-XL width, fp16, 512
 // tokens 145 -> 111 us (fc1 65 -> 59, fc2 with the sum of its pieces 68 -> 40; 273 MB
 // of weights: 45 us at the streaming rate); DiT-G width with fp8 weights, 512 tokens
-// 439 -> 274 us (860 MB: 141 us).  What is left over the streaming time: a
+// 439 -> 255 us (860 MB: 141 us).  What is left over the streaming time: a
 // workgroup's start (row ranges, row table, first copies: 4 to 5 us), the last round
 // of workgroups, and the products, which the lockstep of a workgroup's waves hides
 // only in part.
