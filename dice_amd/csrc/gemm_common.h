@@ -31,6 +31,7 @@ struct GemmParams {
   const int32_t *c_perm;   // grouped row -> output row.  NULL: identity
   int n;                   // output columns
   int k;                   // reduction length
+  int far_slot;            // > 0: only tiles with a row whose slot is this or more (the others hold what another kernel wrote)
 };
 
 struct TileCoord {

@@ -107,6 +107,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *kWave) void grouped_gemm_bf16_ker
   if (!t.active) return;
 
   const int tid = threadIdx.x;
+  if (p.far_slot > 0) {
+    int far = 0;
+    for (int r = tid; r < t.rows_valid; r += NT) far |= p.a_perm[t.row_begin + r] >= p.far_slot;
+    if (!__syncthreads_or(far)) return;
+  }
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;

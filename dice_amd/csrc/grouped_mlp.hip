@@ -303,7 +303,9 @@ extern "C" int dice_grouped_mlp_a8(int stages, const void *x, int act_dtype, con
 
 namespace dice {
 namespace {
-int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *perm,
+// x_rows: rows of x, or kUnknownRows.
+constexpr int64_t kUnknownRows = -1;
+int grouped_mlp_impl(int stages, const void *x, int64_t x_rows, int act_dtype, const int32_t *perm,
                      int slots_per_token, const int32_t *offsets, int n_experts, int64_t max_rows,
                      int hidden, int inter, const void *w1, const float *b1, const void *w2,
                      const float *b2, const float *w1_scale, const float *w2_scale, int w_dtype,
@@ -336,15 +338,19 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
   pb1.n_problems = pb2.n_problems = 1;
   pb1.prob[0] = PersistProblem{x, hidden, offsets, n_experts, w1, swiglu ? 2 * inter : inter, inter,
                                swiglu ? nullptr : b1, h, inter, inter, hidden, (int)max_rows};
+  // The kernels that gather rows through a 2 GiB descriptor (the persistent, streaming and split ones) read
+  // rows past it as zeros.  A source that is known to be larger is refused by their predicates; of one of
+  // unknown size they take what a descriptor covers, and the tiles that hold a slot past it are then
+  // multiplied again by the permutation-addressed kernels, whose offsets go further (far_slot).
+  int64_t far_slot = 0;
   if (perm) {
-    // This entry point is not told how many rows x has: the row addresses get
-    // the widest range the kernel can address (the permutation-addressed
-    // kernel checks none either); slots beyond it fall back to that kernel.
-    pb1.prob[0].a_rows = perm;
-    pb1.prob[0].a_div = slots_per_token;
     const int64_t by_slots = ((1ll << 28) - 1) / slots_per_token;
     const int64_t by_bytes = ((1ll << 31) - 1) / ((int64_t)hidden * dtype_size(act_dtype));
-    pb1.prob[0].a_src_rows = (int)(by_slots < by_bytes ? by_slots : by_bytes);
+    const int64_t covered = by_slots < by_bytes ? by_slots : by_bytes;
+    if (x_rows == kUnknownRows) far_slot = covered * slots_per_token;
+    pb1.prob[0].a_rows = perm;
+    pb1.prob[0].a_div = slots_per_token;
+    pb1.prob[0].a_src_rows = (int)(x_rows == kUnknownRows ? covered : x_rows < INT32_MAX ? x_rows : INT32_MAX);
   }
   pb2.prob[0] = PersistProblem{h, inter, offsets, n_experts, w2, hidden, 0, swiglu ? nullptr : b2,
                                out, hidden, hidden, inter, (int)max_rows};
@@ -365,12 +371,7 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
     s1.tall = s2.tall = stream_tall(max_rows, n_experts);
     streams = stream_supported(s1, m1) && stream_supported(s2, kFc2);
   }
-  if (streams) {
-    rc = stages & 1 ? launch_stream(s1, m1, act_dtype, s) : (int)DICE_OK;
-    if (rc || !(stages & 2)) return rc;
-    return launch_stream(s2, kFc2, act_dtype, s);
-  }
-  if (is_16bit(act_dtype)) {
+  if (!streams && is_16bit(act_dtype)) {
     const bool few = few_rows_per_group(max_rows, n_experts);
     fc1_persist = gemm_config_allows_persistent(m1) && !(few && gemm_config_is_default(m1)) && persist_supported(pb1, m1);
     fc2_persist = !scatter_to_slots && gemm_config_allows_persistent(kFc2) &&
@@ -378,9 +379,12 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
   }
 
   if (stages & 1) {
-    if (fc1_persist) {
+    if (streams)
+      rc = launch_stream(s1, m1, act_dtype, s);
+    else if (fc1_persist)
       rc = launch_persist(pb1, m1, act_dtype, s);
-    } else {
+    if (rc) return rc;
+    if (far_slot > 0 || !(streams || fc1_persist)) {
       GemmParams p1{};
       p1.a = x;
       p1.a_perm = perm;
@@ -398,11 +402,13 @@ int grouped_mlp_impl(int stages, const void *x, int act_dtype, const int32_t *pe
       p1.c_perm = nullptr;
       p1.n = inter;
       p1.k = hidden;
+      if (streams || fc1_persist) p1.far_slot = (int)far_slot;
       rc = run_gemm(p1, m1, act_dtype, w_dtype, max_rows, s);
     }
     if (rc) return rc;
   }
   if (!(stages & 2)) return DICE_OK;
+  if (streams) return launch_stream(s2, kFc2, act_dtype, s);
   if (fc2_persist) return launch_persist(pb2, kFc2, act_dtype, s);
 
   GemmParams p2{};
@@ -434,7 +440,7 @@ extern "C" int dice_grouped_mlp(const void *x, int act_dtype, const int32_t *per
                                 const float *w1_scale, const float *w2_scale, int w_dtype,
                                 int act_variant, void *h, void *out, int scatter_to_slots,
                                 void *stream) {
-  return dice::grouped_mlp_impl(3, x, act_dtype, perm, slots_per_token, offsets, n_experts, max_rows,
+  return dice::grouped_mlp_impl(3, x, dice::kUnknownRows, act_dtype, perm, slots_per_token, offsets, n_experts, max_rows,
                                 hidden, inter, w1, b1, w2, b2, w1_scale, w2_scale, w_dtype,
                                 act_variant, h, out, scatter_to_slots, stream);
 }
@@ -448,7 +454,22 @@ extern "C" int dice_grouped_mlp_stage(int stage, const void *x, int act_dtype, c
                                       void *stream) {
   if (stage != 1 && stage != 2)
     return dice::fail(DICE_ERR_BAD_ARG, "dice_grouped_mlp_stage: stage %d (1 = fc1, 2 = fc2)", stage);
-  return dice::grouped_mlp_impl(stage, x, act_dtype, perm, slots_per_token, offsets, n_experts,
+  return dice::grouped_mlp_impl(stage, x, dice::kUnknownRows, act_dtype, perm, slots_per_token, offsets, n_experts,
+                                max_rows, hidden, inter, w1, b1, w2, b2, w1_scale, w2_scale, w_dtype,
+                                act_variant, h, out, scatter_to_slots, stream);
+}
+
+extern "C" int dice_grouped_mlp_rows(int stages, const void *x, int64_t x_rows, int act_dtype, const int32_t *perm,
+                                     int slots_per_token, const int32_t *offsets, int n_experts,
+                                     int64_t max_rows, int hidden, int inter, const void *w1,
+                                     const float *b1, const void *w2, const float *b2,
+                                     const float *w1_scale, const float *w2_scale, int w_dtype,
+                                     int act_variant, void *h, void *out, int scatter_to_slots,
+                                     void *stream) {
+  if (stages < 1 || stages > 3)
+    return dice::fail(DICE_ERR_BAD_ARG, "dice_grouped_mlp_rows: stages %d (1 = fc1, 2 = fc2, 3 = both)", stages);
+  if (x_rows < 0) return dice::fail(DICE_ERR_BAD_ARG, "dice_grouped_mlp_rows: x_rows %lld", (long long)x_rows);
+  return dice::grouped_mlp_impl(stages, x, x_rows, act_dtype, perm, slots_per_token, offsets, n_experts,
                                 max_rows, hidden, inter, w1, b1, w2, b2, w1_scale, w2_scale, w_dtype,
                                 act_variant, h, out, scatter_to_slots, stream);
 }
@@ -883,13 +904,13 @@ int forward_impl(const char *who, const dice_moe_layer_t *L, const dice_moe_laye
     const bool shared = L->shared_inter > 0;
     for (int stage = 1; stage <= 2; ++stage) {
       stamp(stage == 1 ? 3 : 6, s);
-      rc = grouped_mlp_impl(stage, work.x, L->act_dtype, work.perm, L->top_k, work.offsets, L->n_experts, max_rows,
+      rc = grouped_mlp_impl(stage, work.x, n_tokens, L->act_dtype, work.perm, L->top_k, work.offsets, L->n_experts, max_rows,
                             L->hidden, L->inter, LE->w1, LE->b1, LE->w2, LE->b2, LE->w1_scale, LE->w2_scale,
                             LE->w_dtype, L->act_variant, w.h, work.rows, 0, stream);
       if (rc) return rc;
       stamp(stage == 1 ? 4 : 7, s);
       if (shared) {
-        rc = grouped_mlp_impl(stage, x, L->act_dtype, nullptr, 1, w.shared_offsets, 1, n_tokens, L->hidden,
+        rc = grouped_mlp_impl(stage, x, n_tokens, L->act_dtype, nullptr, 1, w.shared_offsets, 1, n_tokens, L->hidden,
                               L->shared_inter, L->shared_w1, L->shared_b1, L->shared_w2, L->shared_b2, nullptr,
                               nullptr, L->act_dtype, L->act_variant, w.shared_h, w.shared_out, 0, stream);
         if (rc) return rc;

@@ -37,6 +37,7 @@ EXPORTS = [
     "dice_gather_rows",
     "dice_grouped_mlp",
     "dice_grouped_mlp_stage",
+    "dice_grouped_mlp_rows",
     "dice_set_gemm_config",
     "dice_debug_persist_turns",
     "dice_profile_enable",
@@ -128,6 +129,8 @@ def load() -> ctypes.CDLL:
                                      c_int, c_int, c_void_p, c_void_p, c_int, c_void_p]
     lib.dice_grouped_mlp_stage.restype = c_int
     lib.dice_grouped_mlp_stage.argtypes = [c_int] + lib.dice_grouped_mlp.argtypes
+    lib.dice_grouped_mlp_rows.restype = c_int
+    lib.dice_grouped_mlp_rows.argtypes = [c_int, c_void_p, c_int64] + lib.dice_grouped_mlp.argtypes[1:]
     lib.dice_combine.restype = c_int
     lib.dice_combine.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_int, c_int64, c_int, c_int, c_void_p]

@@ -104,8 +104,8 @@ def grouped_mlp(x: torch.Tensor, perm: Optional[torch.Tensor], slots_per_token: 
         h = torch.empty((max(max_rows, 1), inter), dtype=x.dtype, device=x.device)
     if out is None:
         out = torch.zeros((n_out_rows, d), dtype=x.dtype, device=x.device)
-    check(load().dice_grouped_mlp(
-        ptr(x), dtype_code(x.dtype), ptr(perm), slots_per_token, ptr(offsets), e, max_rows, d, inter,
+    check(load().dice_grouped_mlp_rows(
+        3, ptr(x), x.numel() // d, dtype_code(x.dtype), ptr(perm), slots_per_token, ptr(offsets), e, max_rows, d, inter,
         ptr(w1), ptr(b1), ptr(w2), ptr(b2), ptr(w1_scale), ptr(w2_scale), dtype_code(w1.dtype),
         VARIANTS[variant], ptr(h), ptr(out), int(bool(scatter_to_slots)), stream_ptr()))
     return out

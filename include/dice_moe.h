@@ -146,6 +146,10 @@ int dice_gather_rows(const void *x, int dtype, const int32_t *perm,
  * Expert outputs are NOT scaled by the routing weight here (the skip cache
  * stores them unscaled, ep_fwd.py:188); dice_combine applies the weights.
  * Limits: hidden % 64 == 0, inter % 64 == 0, n_experts <= 256.
+ * With perm, x may have any number of rows, which this entry point is not told:
+ * behind fc1 a second launch looks at every tile's slots and multiplies those
+ * again that reach past the 2 GiB of x that the first one covers (a few
+ * microseconds where none does).  dice_grouped_mlp_rows is told and has no such launch.
  */
 int dice_grouped_mlp(const void *x, int act_dtype, const int32_t *perm,
                      int slots_per_token, const int32_t *offsets,
@@ -170,6 +174,18 @@ int dice_grouped_mlp_stage(int stage, const void *x, int act_dtype,
                            const float *w2_scale, int w_dtype, int act_variant,
                            void *h, void *out, int scatter_to_slots,
                            void *stream);
+
+/*
+ * dice_grouped_mlp (stages = 3) or one stage of it (1, 2) with the number of rows
+ * of x: perm[r] / slots_per_token < x_rows.
+ */
+int dice_grouped_mlp_rows(int stages, const void *x, int64_t x_rows, int act_dtype,
+                          const int32_t *perm, int slots_per_token,
+                          const int32_t *offsets, int n_experts, int64_t max_rows,
+                          int hidden, int inter, const void *w1, const float *b1,
+                          const void *w2, const float *b2, const float *w1_scale,
+                          const float *w2_scale, int w_dtype, int act_variant,
+                          void *h, void *out, int scatter_to_slots, void *stream);
 
 /*
  * Combine.  Replaces mul_ by the routing weight + scatter_reduce_ of moe_infer
