@@ -10,8 +10,18 @@
 // the rounding of one addition.  (The decomposition is the classical one for products
 // in higher precision from lower-precision parts: T. J. Dekker, Numer. Math. 18, 1971.)
 // Against float64 the rows are as close as those of the fp32 matrix instructions, whose
-// sum is rounded at every second product, here six times in sixteen.  A value that
-// rounds to infinity in bf16 (above 3.39e38) makes the elements it enters NaN.
+// sum is rounded at every second product, here six times in sixteen.
+//
+// Operands that three parts do not represent: infinities and what rounds to infinity in
+// bf16 (above 3.39e38; the remainders are then infinity less infinity), and magnitudes
+// below about 2^-110, whose third part falls out of bf16's range.  The first make a sum
+// that is not finite, the second, among their like, a small one.  A lane that finds such
+// a sum in its row (see represented) forms the row's sums of its tile again in the epilogue,
+// as fp32 sums of fp32 products.  What stays is a factor below 2^-110, good to 2^-134,
+// beside one of 2^40 and more.  The check costs one instruction per sum: 0.1 us of a launch
+// at DiT-S width, nothing that shows at DiT-B (written as four, 21 of 1540 us); 8192 tokens
+// of DiT-B width take 23 ms where every sum is formed again, 3.7 with an infinity in one
+// token.
 //
 // A workgroup multiplies BM grouped rows x BN weight rows.  Rows travel as whole
 // 128-byte lines (32 k) through registers, STAGES lines ahead; a thread holds pairs of
@@ -81,6 +91,29 @@ __device__ __forceinline__ Parts split_pair(float x, float y, uint32_t minus_lo,
   y = less_half(y, p.b, minus_hi);
   p.c = round_pair(x, y);
   return p;
+}
+
+// Whether sums of the magnitudes lo .. hi (or NaN) are what the parts give: all finite (an operand that is infinite
+// or rounds to infinity in bf16 leaves no number), and none so small that operands may have been below the range
+// of their third part.  An exact zero is not doubtful, and the caller leaves it out.
+__device__ __forceinline__ bool represented(float lo, float hi) { return lo >= 0x1p-64f && hi < __builtin_inff(); }
+// The sums of `x` with the N weight rows at w, w + stride .. in fp32, one product at a time.
+template <int N>
+__device__ __forceinline__ void plain_sums(const float *x, const float *w, size_t stride, int k, float *sum) {
+#pragma unroll
+  for (int r = 0; r < N; ++r) sum[r] = 0.f;
+  for (int i = 0; i < k; i += 4) {
+    const f32x4_t xv = *reinterpret_cast<const f32x4_t *>(x + i);
+    bool nan = true;
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      const f32x4_t wv = *reinterpret_cast<const f32x4_t *>(w + r * stride + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[r] = __builtin_fmaf(xv[e], wv[e], sum[r]);
+      nan = nan && __builtin_isnan(sum[r]);
+    }
+    if (nan) break;   // (stays one)
+  }
 }
 
 template <typename G>
@@ -235,8 +268,45 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
     if constexpr (LIVE > 0) {
       constexpr int BW = SWIGLU ? 16 : 32;   // output columns of a weight block
       const float *bias = p.bias ? p.bias + (size_t)t.expert * n : nullptr;
+      auto activate = [](float x, float up, float bias_v) {
+        if (SWIGLU) return silu_fast(x) * up;
+        x += bias_v;
+        return MODE == kFc1Gelu ? gelu_tanh_fast(x) : x;
+      };
       float *const out = (float *)p.c + (size_t)(t.pieces > 1 ? t.piece : 0) * p.max_rows * p.ldc;
       size_t dst[LV];
+      // Bit i of redo: this lane's row of row block i has such a sum.  First by the smallest and the largest
+      // magnitude (one instruction per sum; both propagate NaN), which exact zeros can make look closer.
+      uint32_t redo = 0;
+      float hi[LV];
+#pragma unroll
+      for (int i = 0; i < LIVE; ++i) {
+        float lo = 1.f;
+        hi[i] = 1.f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; e += 2) {
+            const float a = __builtin_fabsf(acc[i][j][e]), c = __builtin_fabsf(acc[i][j][e + 1]);
+            lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(a, c), lo);
+            hi[i] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, c), hi[i]);
+          }
+        redo |= represented(lo, hi[i]) || (i * WM + wm) * 32 + frag_row >= t.rows ? 0u : 1u << i;
+      }
+      if (__any(redo != 0)) {
+#pragma unroll
+        for (int i = 0; i < LIVE; ++i) {
+          float lo = 1.f;
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              const float a = __builtin_fabsf(acc[i][j][e]);
+              lo = __builtin_elementwise_minimum(a == 0.f ? 1.f : a, lo);
+            }
+          redo &= represented(lo, hi[i]) ? ~(1u << i) : ~0u;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < LV; ++i) {
         const int m = (i * WM + wm) * 32 + frag_row;
@@ -255,19 +325,36 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
             const int m = (i * WM + wm) * 32 + frag_row;
             f32x4_t v;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              float x = acc[i][j][q * 4 + r];
-              if (SWIGLU) {
-                x = silu_fast(x) * acc[i][j][8 + q * 4 + r];
-              } else {
-                x += sb[r];
-                if (MODE == kFc1Gelu) x = gelu_tanh_fast(x);
-              }
-              v[r] = x;
-            }
+            for (int r = 0; r < 4; ++r)
+              v[r] = activate(acc[i][j][q * 4 + r], SWIGLU ? acc[i][j][8 + q * 4 + r] : 1.f, SWIGLU ? 0.f : sb[r]);
             if (m < t.rows && col < n) *reinterpret_cast<f32x4_t *>(out + dst[i] + col) = v;
           }
         }
+      // These rows are formed again, whole, as fp32 sums (by the lane that wrote them).  Only operands at the ends of
+      // the fp32 range get here.
+      if (__any(redo != 0)) {
+#pragma unroll 1
+        for (int i = 0; i < LIVE; ++i) {
+          if ((redo >> i & 1) == 0) continue;
+          const int m = (i * WM + wm) * 32 + frag_row;
+          const size_t src = p.a_rows ? (size_t)(p.a_rows[t.row0 + m] / p.a_div) : (size_t)(t.row0 + m);
+          const float *const x = (const float *)p.a + src * p.lda + line0 * 32;
+          float *const row = out + (size_t)(b.c_rows ? b.c_rows[t.row0 + m] : t.row0 + m) * p.ldc;
+#pragma unroll 1
+          for (int c = 0; c < TN * (BW / 8); ++c) {
+            const int col = t.n0 + (wn * TN + c / (BW / 8)) * BW + half * 4 + c % (BW / 8) * 8;
+            if (col >= n) continue;
+            const float *const w = (const float *)p.w + ((size_t)t.expert * p.w_rows + col) * k + line0 * 32;
+            float sum[4], up[4] = {1.f, 1.f, 1.f, 1.f};
+            plain_sums<4>(x, w, k, lines * 32, sum);
+            if (SWIGLU) plain_sums<4>(x, w + (size_t)p.up_offset * k, k, lines * 32, up);
+            f32x4_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = activate(sum[r], up[r], !SWIGLU && bias && t.piece == 0 ? bias[col + r] : 0.f);
+            *reinterpret_cast<f32x4_t *>(row + col) = v;
+          }
+        }
+      }
     }
   };
   if constexpr (TM >= 4) {
