@@ -17,8 +17,9 @@
 // below about 2^-110, whose third part falls out of bf16's range.  The first make a sum
 // that is not finite, the second, among their like, a small one.  A lane that finds such
 // a sum in its row (see represented) forms the row's sums of its tile again in the epilogue,
-// as fp32 sums of fp32 products.  What stays is a factor below 2^-110, good to 2^-134,
-// beside one of 2^40 and more.  The check costs one instruction per sum: 0.1 us of a launch
+// as fp32 sums of fp32 products.  What stays: a factor below 2^-110 is good to 2^-134
+// in a sum that passes 2^-64 all the same, and a sum whose products all have a factor
+// below 2^-134 is zero.  The check costs one instruction per sum: 0.1 us of a launch
 // at DiT-S width, nothing that shows at DiT-B (written as four, 21 of 1540 us); 8192 tokens
 // of DiT-B width take 23 ms where every sum is formed again, 3.7 with an infinity in one
 // token.

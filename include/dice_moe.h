@@ -147,9 +147,9 @@ int dice_gather_rows(const void *x, int dtype, const int32_t *perm,
  * stores them unscaled, ep_fwd.py:188); dice_combine applies the weights.
  * Limits: hidden % 64 == 0, inter % 64 == 0, n_experts <= 256.
  * F32 products are formed from bf16 parts where the kernels for that apply, with
- * the error of fp32 sums; infinities, NaN and subnormal values propagate as in
- * fp32.  A factor below 2^-110 is good to 2^-134 where the sum it enters is above
- * 2^-64.
+ * the error of fp32 sums; infinities and NaN propagate as in fp32.  A factor below
+ * 2^-110 is good to 2^-134 where the sum it enters is above 2^-64, and a sum whose
+ * products all have a factor below 2^-134 is zero.
  * With perm, x may have any number of rows, which this entry point is not told:
  * behind fc1 a second launch looks at every tile's slots and multiplies those
  * again that reach past the 2 GiB of x that the first one covers (a few
