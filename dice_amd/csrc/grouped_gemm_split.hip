@@ -6,11 +6,17 @@
 // bf16 numbers, every one exact in the matrix pipe's fp32 accumulator.  Six are formed,
 // the smallest first:
 //   a3 b1, a2 b2, a1 b3, a2 b1, a1 b2, a1 b1;
-// the three left out are together below 2^-25 of the product, of either sign: less than
-// the rounding of one addition.  (The decomposition is the classical one for products
+// the three left out are together at most 2^-24 of the product (a2 <= 2^-8, a3 <= 2^-17 of
+// the leading bit's value; a = b = 1.0038986 comes to 0.99 of it), of either sign: the size
+// of one rounding.  (The decomposition is the classical one for products
 // in higher precision from lower-precision parts: T. J. Dekker, Numer. Math. 18, 1971.)
-// Against float64 the rows are as close as those of the fp32 matrix instructions, whose
-// sum is rounded at every second product, here six times in sixteen.
+//
+// Against float64, beside the fp32 matrix instructions, which round their sum at every
+// second product where these do six times in sixteen (and not always to nearest: a sum
+// of one product is off by up to 2.5 x 2^-24, theirs by 1): rows of fc1 and fc2 at DiT-S
+// and DiT-B width have relative errors of 3.4e-7 to 8.6e-7 against 4.1e-7 to 9.9e-7.  Rows
+// that are zero for the most part have larger ones than there, whose zeros round nothing: 1.3
+// x with one product that is not zero in 512, 2.2 x with 16, 1.6 x with 64.
 //
 // Operands that three parts do not represent: infinities and what rounds to infinity in
 // bf16 (above 3.39e38; the remainders are then infinity less infinity), and magnitudes
@@ -19,8 +25,8 @@
 // a sum in its row (see represented) forms the row's sums of its tile again in the epilogue,
 // as fp32 sums of fp32 products.  What stays: a factor below 2^-110 is good to 2^-134
 // in a sum that passes 2^-64 all the same, and a sum whose products all have a factor
-// below 2^-134 is zero.  The check costs one instruction per sum: 0.1 us of a launch
-// at DiT-S width, nothing that shows at DiT-B (written as four, 21 of 1540 us); 8192 tokens
+// below 2^-134 is zero.  The check costs one instruction per sum: 0.1 to 0.2 us of a
+// launch at DiT-S width, nothing that shows at DiT-B (written as four, 21 of 1540 us); 8192 tokens
 // of DiT-B width take 23 ms where every sum is formed again, 3.7 with an infinity in one
 // token.
 //

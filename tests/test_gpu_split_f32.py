@@ -28,7 +28,7 @@ def _rel(got, want):
     return float((got.double() - want).norm() / want.norm())
 
 
-# rows per expert; the last column is the tile the two stages take
+# rows per expert; the comments name the tiles that the two stages take
 @pytest.mark.parametrize("counts,D,I,variant", [
     ([1], 64, 64, "swiglu"),                            # 64 x 64; one row, two lines of k
     ([63, 0, 64, 65], 128, 192, "gelu_tanh"),           # 64 x 64; around a tile, an expert without rows
@@ -92,3 +92,41 @@ def test_layer_with_cut_fc2(dev, N, D, E, k, ratio):
         cache = torch.empty_like(x)
         assert torch.equal(y, blk.run(x, lib.MODE_PUT, mask, None, cache))
         assert torch.equal(y, blk.run(x, lib.MODE_SKIP, mask, cache, None))
+
+
+def _parts(v):
+    a = v.bfloat16().float()
+    b = (v - a).bfloat16().float()
+    return a.double(), b.double(), (v - a - b).double()
+
+
+@pytest.mark.parametrize("products", [1, 2])
+def test_sums_of_few_products(dev, products):
+    """Where nothing averages out: one or two products that are not zero.  The parts left out are at most 2^-24 of a
+    product.  An addition of the matrix pipe is good to an ulp of its sum (2^-23): the last of the first product's six
+    (those before it act on sums of at most 2^-6), all six of the second's."""
+    from dice_amd import lib
+    K, N, R = 512, 256, 300
+    g = torch.Generator().manual_seed(products)
+    v = 1 + torch.rand(R, generator=g)
+    v[:8] = 1.0038986   # (next to the worst pair: parts of 2^-8 and 2^-17)
+    h = torch.zeros(R, K)
+    at = torch.randint(0, K // products, (R,), generator=g)
+    for i in range(products):
+        h[torch.arange(R), at + i * (K // products)] = v.roll(i)
+    w = (1 + torch.rand(N, K, generator=g)) * (1 - 2 * (torch.rand(N, K, generator=g) < 0.5).float())
+    w[:16] = 1.0038986
+    # the parts themselves
+    a, b, c = _parts(torch.cat([v, w.reshape(-1)]))
+    whole = torch.cat([v, w.reshape(-1)]).double()
+    assert torch.equal(a + b + c, whole) and torch.equal(c, c.float().bfloat16().double())
+    lost = 2 * b.abs() * c.abs() + c * c
+    assert float((lost / (whole * whole)).max()) <= 2.0 ** -24 * (1 + 2.0 ** -8)
+    out = torch.empty(R, N, device=dev)
+    hd, wd, off = h.to(dev), w.to(dev), torch.tensor([0, R], dtype=torch.int32, device=dev)
+    p = lib.ptr
+    lib.check(lib.load().dice_grouped_mlp_rows(2, p(hd), R, 0, None, 1, p(off), 1, R, N, K, p(wd), None, p(wd), None,
+                                               None, None, 0, 0, p(hd), p(out), 0, lib.stream_ptr()))
+    want, size = h.double() @ w.double().t(), h.double() @ w.double().abs().t()
+    bound = 2.0 ** -24 * (1 + 2 * (1 + 6 * (products - 1)) + 2.0 ** -3) * size
+    assert bool(((out.cpu().double() - want).abs() <= bound).all())
