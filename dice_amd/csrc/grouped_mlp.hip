@@ -517,8 +517,11 @@ bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_r
 // beside uncut routed tiles they were its last turn (layer call, shared fc2 whole
 // / cut, us: DiT-G width, fp8 weights, 512 tokens, SwiGLU (k = 4096) 268 / 257, GELU
 // (k = 16384) 371 / 254; width 1408, 16 experts, GELU, 800 tokens 245 / 217).
-// Whether and how far depends on the layer's shape alone, not on the batch, so
-// that a skip step and the full step it belongs to add up their rows alike.
+// How far depends on the layer's shape alone, not on the batch, so that a skip step and
+// the full step it belongs to add up their rows alike where both stream.  Whether a step
+// does depends on its rows, of which a skip step has half: at DiT-XL width (SwiGLU, 8
+// experts) between 961 and 1920 tokens only the skip step streams, and its rows then
+// differ from the full step's by what the latter rounds to 16 bits before the combine.
 StreamPlan plan_stream(const dice_moe_layer_t *L, const dice_moe_layer_t *LE, int64_t n_tokens, int64_t max_rows) {
   StreamPlan plan{false, false, 1, 1};
   if (L->act_dtype == DICE_F32) {

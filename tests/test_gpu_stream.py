@@ -101,11 +101,14 @@ def test_fp8_weights_on_the_streaming_kernels(dev, N, D, E, ratio, variant):
     check_rows(y.cpu().view(-1, D), other.cpu().view(-1, D), 8e-3, "fp8 weights, streaming vs persistent")
 
 
-def test_put_and_skip_on_partial_rows(dev):
+@pytest.mark.parametrize("N", [320, 960, 961, 1920])
+def test_put_and_skip_on_partial_rows(dev, N):
     """A put step writes the rows that its combine added up from pieces; a skip
-    step, cut alike, reproduces the put step's output from them bit for bit."""
+    step, cut alike, reproduces the put step's output from them bit for bit.  From
+    961 tokens on the put step takes the persistent kernels, whose rows are rounded
+    before they are combined, and the skip step alone streams."""
     from dice_amd import lib
-    D, N = 1152, 320
+    D = 1152
     p = _params(D, 8, 2, 4, "swiglu", torch.bfloat16, 5)
     x = torch.randn(N, D, generator=torch.Generator().manual_seed(6)).bfloat16().to(dev)
     blk = block_from_params(p, D, "swiglu", torch.bfloat16, dev)
@@ -113,7 +116,11 @@ def test_put_and_skip_on_partial_rows(dev):
     cache = torch.empty_like(x)
     put = blk.run(x, lib.MODE_PUT, mask, None, cache).clone()
     assert torch.equal(put, blk.run(x))
-    assert torch.equal(put, blk.run(x, lib.MODE_SKIP, mask, cache, None))
+    skip = blk.run(x, lib.MODE_SKIP, mask, cache, None)
+    if N <= 960:
+        assert torch.equal(put, skip)
+    else:   # (a rounding of 2^-9 of the row that is not cached and one of the sum)
+        check_rows(skip.cpu(), put.cpu(), 2.0 ** -8, "skip step on its own cache")
 
 
 def test_entry_with_few_rows_in_a_large_batch(dev):
