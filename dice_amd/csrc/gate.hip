@@ -262,7 +262,6 @@ int launch_gate(const void *x, const void *w, const float *bias, int64_t n_token
   return launch_status("dice_gate_topk");
 }
 
-
 // ---------------------------------------------------------------------------
 // The router on the matrix pipe (16-bit activations and router matrix, at most
 // 32 experts).  The kernel above spends its time issuing instructions - about
@@ -461,7 +460,7 @@ int launch_gate_mfma(const void *x, const void *w, const float *bias, int64_t n_
 // 8.4e-8 at 384, 9.1e-8 / 9.3e-8 at 768, 1.04e-7 / 1.06e-7 at 1152.
 constexpr int kRouterF32Chunks = 18;   // per wave: 16 floats of a row each
 constexpr int kRouterF32Waves = 4;
-__device__ __forceinline__ void gate_topk_f32_body(
+__global__ __launch_bounds__(kRouterF32Waves *kWave) void gate_topk_f32_kernel(
     const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias, int64_t n_tokens,
     int hidden, int n_experts, int top_k, int norm_topk, int32_t *__restrict__ topk_idx,
     int64_t *__restrict__ topk_idx64, float *__restrict__ topk_weight, float *__restrict__ logits_out) {
@@ -577,13 +576,6 @@ __device__ __forceinline__ void gate_topk_f32_body(
       topk_weight[tok * top_k + j] = (norm_topk && top_k > 1) ? sel_w[r] / (picked_sum + 1e-20f) : sel_w[r];
     }
   }
-}
-__global__ __launch_bounds__(kRouterF32Waves *kWave) void gate_topk_f32_kernel(
-    const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias, int64_t n_tokens,
-    int hidden, int n_experts, int top_k, int norm_topk, int32_t *__restrict__ topk_idx,
-    int64_t *__restrict__ topk_idx64, float *__restrict__ topk_weight, float *__restrict__ logits_out) {
-  gate_topk_f32_body(x, w, bias, n_tokens, hidden, n_experts, top_k, norm_topk, topk_idx, topk_idx64, topk_weight,
-                     logits_out);
 }
 
 // ---------------------------------------------------------------------------

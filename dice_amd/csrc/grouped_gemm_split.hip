@@ -68,6 +68,7 @@ struct SplitGeom {
   static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BN_OUT = SWIGLU ? BN / 2 : BN;
   static constexpr int ROWS = BM + BN, PASS_ROWS = WAVES * 16;   // rows of a load pass (four threads each)
   static constexpr int A_PASSES = BM / PASS_ROWS, PASSES = ROWS / PASS_ROWS;
+  static_assert(TM <= 2 && STAGES <= 2, "what split_body has a case for");
   static_assert(BM % PASS_ROWS == 0 && BN % PASS_ROWS == 0, "whole passes of either operand");
   static constexpr int PLANE = ROWS * 32, BUFFER = 3 * PLANE;
   static constexpr size_t LDS = 2 * BUFFER;
@@ -259,16 +260,10 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
     int l = 0;
     for (; l + STAGES <= lines; l += STAGES) {
       line(l, int_c<0>{});
-      if constexpr (STAGES > 1) line(l + 1, int_c<1 % STAGES>{});
-      if constexpr (STAGES > 2) line(l + 2, int_c<2 % STAGES>{});
-      if constexpr (STAGES > 3) line(l + 3, int_c<3 % STAGES>{});
+      if constexpr (STAGES == 2) line(l + 1, int_c<1>{});
     }
-    if constexpr (STAGES > 1) {
+    if constexpr (STAGES == 2) {
       if (l < lines) line(l, int_c<0>{});
-    }
-    if constexpr (STAGES > 2) {
-      if (l + 1 < lines) line(l + 1, int_c<1>{});
-      if (l + 2 < lines) line(l + 2, int_c<2 % STAGES>{});
     }
 
     // ---- epilogue: lane holds row frag_row, columns 8 q + 4 half + {0..3} of each block ----
@@ -364,11 +359,7 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
       }
     }
   };
-  if constexpr (TM >= 4) {
-    if (live >= 4) return run(int_c<4>{});
-    if (live >= 3) return run(int_c<3>{});
-  }
-  if constexpr (TM >= 2) {
+  if constexpr (TM == 2) {
     if (live >= 2) return run(int_c<2>{});
   }
   if (live >= 1) return run(int_c<1>{});

@@ -105,6 +105,7 @@ struct StreamGeom {
   static constexpr int PITCH = BN_OUT * 2 + 16;   // bytes of a staged output row
   static constexpr size_t RINGS = (size_t)SA * A_SLOT + (size_t)SW * W_SLOT, STAGED = (size_t)BM * PITCH;
   static constexpr size_t LDS = RINGS > STAGED ? RINGS : STAGED;
+  static_assert(TM == 2 || TM == 3, "what stream_body has a case for");
   static_assert(SW > 2 || SA == 2, "the refill order follows the rings' depth");
   static_assert(SA >= 2 && A_COPIES >= 1 && W_COPIES >= 1 && A_COPIES <= 24 && W_COPIES <= 24, "copies per wave");
   static_assert(A_COPIES * (WAVES / 2) * COPY_ROWS == BM * A_SUB && W_COPIES * (WAVES / 2) * COPY_ROWS == BN, "whole copies");
@@ -367,21 +368,10 @@ __device__ __forceinline__ void stream_body(const StreamBatch &b, const StreamTi
       }
     }
   };
-  if constexpr (TM >= 6) {
-    if (live >= 6) return run(int_c<6>{});
-  }
-  if constexpr (TM >= 5) {
-    if (live == 5) return run(int_c<5>{});
-  }
-  if constexpr (TM >= 4) {
-    if (live == 4) return run(int_c<4>{});
-  }
-  if constexpr (TM >= 3) {
+  if constexpr (TM == 3) {
     if (live == 3) return run(int_c<3>{});
   }
-  if constexpr (TM >= 2) {
-    if (live == 2) return run(int_c<2>{});
-  }
+  if (live == 2) return run(int_c<2>{});
   if (live >= 1) return run(int_c<1>{});
   run(int_c<0>{});
 }
@@ -459,27 +449,28 @@ bool stream_supported(const StreamBatch &b, int mode) {
 // steps of 16-bit weights measured slower: what limits a step is how much
 // independent work a compute unit has behind its barriers.
 int DICE_STREAM_LAUNCH(const StreamBatch &b, int mode, hipStream_t s) {
-  using Fc1 = Shape<false, 128, 2, 1, 2, 4, 2, 2>;
-  using Fc1Tall = Shape<false, 128, 3, 1, 2, 4, 2, 2>;
-  using Fc1W8 = Shape<true, 64, 2, 2, 2, 4, 2, 3>;
-  using Fc2 = Shape<false, 128, 2, 1, 2, 4, 3, 5>;
-  using Fc2Tall = Shape<false, 128, 3, 1, 2, 4, 3, 4>;
-  using Fc2W8 = Shape<true, 128, 2, 1, 2, 4, 3, 4>;
-  using Fc2W8Pair = Shape<true, 64, 2, 1, 2, 4, 3, 4>;   // (two per compute unit)
+  // (Pair..: two workgroups per compute unit, fc1's and those of an fc2 of more than a turn; Deep..: one)
+  using Pair = Shape<false, 128, 2, 1, 2, 4, 2, 2>;
+  using PairTall = Shape<false, 128, 3, 1, 2, 4, 2, 2>;
+  using PairW8Fc1 = Shape<true, 64, 2, 2, 2, 4, 2, 3>;
+  using Deep = Shape<false, 128, 2, 1, 2, 4, 3, 5>;
+  using DeepTall = Shape<false, 128, 3, 1, 2, 4, 3, 4>;
+  using DeepW8 = Shape<true, 128, 2, 1, 2, 4, 3, 4>;
+  using PairW8Fc2 = Shape<true, 64, 2, 1, 2, 4, 3, 4>;
   const bool w8 = b.prob[0].w_scale != nullptr;
   switch (mode) {
     case kFc1Swiglu:
-      return w8 ? launch_shape<kFc1Swiglu, Fc1W8, Fc1Tall>(b, s)
-                : b.tall ? launch_shape<kFc1Swiglu, Fc1Tall>(b, s) : launch_shape<kFc1Swiglu, Fc1>(b, s);
+      return w8 ? launch_shape<kFc1Swiglu, PairW8Fc1, PairTall>(b, s)
+                : b.tall ? launch_shape<kFc1Swiglu, PairTall>(b, s) : launch_shape<kFc1Swiglu, Pair>(b, s);
     case kFc1Gelu:
-      return w8 ? launch_shape<kFc1Gelu, Fc1W8, Fc1Tall>(b, s)
-                : b.tall ? launch_shape<kFc1Gelu, Fc1Tall>(b, s) : launch_shape<kFc1Gelu, Fc1>(b, s);
+      return w8 ? launch_shape<kFc1Gelu, PairW8Fc1, PairTall>(b, s)
+                : b.tall ? launch_shape<kFc1Gelu, PairTall>(b, s) : launch_shape<kFc1Gelu, Pair>(b, s);
     default:
       if (expected_stream_tiles(b, b.tall && !w8 ? 192 : 128, w8 || b.tall ? 192 : 128, 128) > persist_cu_count())
-        return w8 ? launch_shape<kFc2, Fc2W8Pair, Fc1Tall>(b, s)
-                  : b.tall ? launch_shape<kFc2, Fc1Tall>(b, s) : launch_shape<kFc2, Fc1>(b, s);
-      return w8 ? launch_shape<kFc2, Fc2W8, Fc2Tall>(b, s)
-                : b.tall ? launch_shape<kFc2, Fc2Tall>(b, s) : launch_shape<kFc2, Fc2>(b, s);
+        return w8 ? launch_shape<kFc2, PairW8Fc2, PairTall>(b, s)
+                  : b.tall ? launch_shape<kFc2, PairTall>(b, s) : launch_shape<kFc2, Pair>(b, s);
+      return w8 ? launch_shape<kFc2, DeepW8, DeepTall>(b, s)
+                : b.tall ? launch_shape<kFc2, DeepTall>(b, s) : launch_shape<kFc2, Deep>(b, s);
   }
 }
 
