@@ -21,14 +21,13 @@
 // Operands that three parts do not represent: infinities and what rounds to infinity in
 // bf16 (above 3.39e38; the remainders are then infinity less infinity), and magnitudes
 // below about 2^-110, whose third part falls out of bf16's range.  The first make a sum
-// that is not finite, the second, among their like, a small one.  A lane that finds such
-// a sum in its row (see represented) forms the row's sums of its tile again in the epilogue,
-// as fp32 sums of fp32 products.  What stays: a factor below 2^-110 is good to 2^-134
+// that is not finite, the second, among their like, a small one.  Such a sum (see
+// represented) is formed again in the epilogue, by the lane that holds it, as an fp32 sum of
+// fp32 products.  What stays: a factor below 2^-110 is good to 2^-134
 // in a sum that passes 2^-64 all the same, and a sum whose products all have a factor
-// below 2^-134 is zero.  The check costs one instruction per sum: 0.1 to 0.2 us of a
-// launch at DiT-S width, nothing that shows at DiT-B (written as four, 21 of 1540 us); 8192 tokens
-// of DiT-B width take 23 ms where every sum is formed again, 3.7 with an infinity in one
-// token.
+// below 2^-134 is zero.  The check is one instruction per sum and shows in no
+// launch (as four it cost 21 of 1540 us at DiT-B width).  8192 tokens of DiT-B width take 23
+// ms where every sum is formed again, 3.6 with an infinity in one token.
 //
 // A workgroup multiplies BM grouped rows x BN weight rows.  Rows travel as whole
 // 128-byte lines (32 k) through registers, STAGES lines ahead; a thread holds pairs of
@@ -277,36 +276,38 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
       };
       float *const out = (float *)p.c + (size_t)(t.pieces > 1 ? t.piece : 0) * p.max_rows * p.ldc;
       size_t dst[LV];
-      // Bit i of redo: this lane's row of row block i has such a sum.  First by the smallest and the largest
-      // magnitude (one instruction per sum; both propagate NaN), which exact zeros can make look closer.
-      uint32_t redo = 0;
-      float hi[LV];
+      // Bit 16 (j % 2) + e of redo[i][j / 2]: sum e of block (i, j) is not what the parts give.  First by a row's
+      // smallest and largest magnitude (one instruction per sum; both propagate NaN), which exact zeros can make
+      // look closer.
+      uint32_t redo[LV][(TN + 1) / 2] = {};
+      bool closer = false;
 #pragma unroll
       for (int i = 0; i < LIVE; ++i) {
-        float lo = 1.f;
-        hi[i] = 1.f;
+        float lo = 1.f, hi = 1.f;
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
           for (int e = 0; e < 16; e += 2) {
             const float a = __builtin_fabsf(acc[i][j][e]), c = __builtin_fabsf(acc[i][j][e + 1]);
             lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(a, c), lo);
-            hi[i] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, c), hi[i]);
+            hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, c), hi);
           }
-        redo |= represented(lo, hi[i]) || (i * WM + wm) * 32 + frag_row >= t.rows ? 0u : 1u << i;
+        closer = closer || (!represented(lo, hi) && (i * WM + wm) * 32 + frag_row < t.rows);
       }
-      if (__any(redo != 0)) {
+      closer = __any(closer);
+      if (closer) {
 #pragma unroll
         for (int i = 0; i < LIVE; ++i) {
-          float lo = 1.f;
+          const bool row = (i * WM + wm) * 32 + frag_row < t.rows;
 #pragma unroll
           for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
               const float a = __builtin_fabsf(acc[i][j][e]);
-              lo = __builtin_elementwise_minimum(a == 0.f ? 1.f : a, lo);
+              redo[i][j / 2] |= represented(a == 0.f ? 1.f : a, a) ? 0u : 1u << (j % 2 * 16 + e);
             }
-          redo &= represented(lo, hi[i]) ? ~(1u << i) : ~0u;
+#pragma unroll
+          for (int j = 0; j < TN; j += 2) redo[i][j / 2] = row ? redo[i][j / 2] : 0u;
         }
       }
 #pragma unroll
@@ -332,28 +333,28 @@ __device__ __forceinline__ void split_body(const StreamBatch &b, unsigned char *
             if (m < t.rows && col < n) *reinterpret_cast<f32x4_t *>(out + dst[i] + col) = v;
           }
         }
-      // These rows are formed again, whole, as fp32 sums (by the lane that wrote them).  Only operands at the ends of
-      // the fp32 range get here.
-      if (__any(redo != 0)) {
-#pragma unroll 1
+      // These are formed again as fp32 sums (by the lane that wrote them).  Only operands at the ends of the fp32
+      // range get here.
+      if (closer) {
+#pragma unroll
         for (int i = 0; i < LIVE; ++i) {
-          if ((redo >> i & 1) == 0) continue;
           const int m = (i * WM + wm) * 32 + frag_row;
-          const size_t src = p.a_rows ? (size_t)(p.a_rows[t.row0 + m] / p.a_div) : (size_t)(t.row0 + m);
-          const float *const x = (const float *)p.a + src * p.lda + line0 * 32;
-          float *const row = out + (size_t)(b.c_rows ? b.c_rows[t.row0 + m] : t.row0 + m) * p.ldc;
 #pragma unroll 1
           for (int c = 0; c < TN * (BW / 8); ++c) {
-            const int col = t.n0 + (wn * TN + c / (BW / 8)) * BW + half * 4 + c % (BW / 8) * 8;
-            if (col >= n) continue;
+            const int j = c / (BW / 8), q = c % (BW / 8), col = t.n0 + (wn * TN + j) * BW + half * 4 + q * 8;
+            const uint32_t word = TN > 2 && j >= 2 ? redo[i][(TN - 1) / 2] : redo[i][0], sums = word >> (j % 2 * 16);
+            const uint32_t pick = (SWIGLU ? sums >> q * 4 | sums >> (8 + q * 4) : sums >> q * 4) & 15;
+            if (pick == 0 || col >= n) continue;
+            const size_t src = p.a_rows ? (size_t)(p.a_rows[t.row0 + m] / p.a_div) : (size_t)(t.row0 + m);
+            const float *const x = (const float *)p.a + src * p.lda + line0 * 32;
             const float *const w = (const float *)p.w + ((size_t)t.expert * p.w_rows + col) * k + line0 * 32;
             float sum[4], up[4] = {1.f, 1.f, 1.f, 1.f};
             plain_sums<4>(x, w, k, lines * 32, sum);
             if (SWIGLU) plain_sums<4>(x, w + (size_t)p.up_offset * k, k, lines * 32, up);
-            f32x4_t v;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = activate(sum[r], up[r], !SWIGLU && bias && t.piece == 0 ? bias[col + r] : 0.f);
-            *reinterpret_cast<f32x4_t *>(row + col) = v;
+            for (int r = 0; r < 4; ++r)
+              if (pick >> r & 1)
+                out[dst[i] + col + r] = activate(sum[r], up[r], !SWIGLU && bias && t.piece == 0 ? bias[col + r] : 0.f);
           }
         }
       }

@@ -87,11 +87,7 @@ def test_infinite_weight(dev, counts, D, I):
     same = torch.ones_like(h, dtype=torch.bool)
     same[:n, 5] = False
     same[2] = False
-    # (rows that hold a doubtful sum are formed again whole, in another order)
-    bound = 1.2 * (D + 8) * 2.0 ** -24 * (x[:n].abs().double() @ w1[0].abs().double().t())
-    bound[:, 5] = INF
-    assert bool(((h[:n] - clean_h[:n]).abs().double() <= 2 * bound)[same[:n]].all())
-    assert torch.equal(h[n:], clean_h[n:])
+    assert torch.equal(h[same], clean_h[same])
 
 
 @pytest.mark.parametrize("counts,D,I", SHAPES[:2])
