@@ -38,12 +38,13 @@
 // value against six products of 32 cycles per 32 x 32 x 16 block.  One barrier per
 // sub-step.
 //
-// Bound: large shapes by the matrix pipe under the power limit (256 x 256 tiles: 208
-// TFLOP/s of fp32 products, 1250 of bf16 ones, 14 % faster on zero operands; the fp32
-// instructions reached 116-125), small ones by the chain load - split - LDS - product of
-// a sub-step (about 0.3 us), whatever the tile, the depth of the prefetch or the order
-// of the instructions.  Both stages of DiT-B width (8192 tokens, shared expert
-// included) 2470 -> 1510 us; of DiT-S width, 256 tokens, 105 -> 39 us.
+// Bound: large shapes by the matrix pipe, which is busy for three fifths of the cycles at
+// 1.8 GHz (8192 tokens of DiT-B width: 256 x 256 tiles 181 TFLOP/s of fp32 products, 1085 of
+// bf16 ones, 256 x 128 tiles 173; 10 and 20 % faster on zero weights, which the power limit
+// clocks higher; the fp32 instructions reached 116-125), small ones by the chain load -
+// split - LDS - product of a sub-step (about 0.3 us), whatever the tile, the depth of the
+// prefetch or the order of the instructions.  Layer call at DiT-B width 2490 -> 1510 us,
+// at DiT-S width, 256 tokens, 115 -> 49 us.
 #include <cmath>
 #include <type_traits>
 

@@ -1,9 +1,10 @@
 // Grouped expert GEMMs for small batches, where a launch is the streaming of its
-// weights: an expert has few rows (up to about 190, in layer calls somewhat more), every weight is multiplied with
-// them once, and what counts is that weight bytes are in flight on every compute
-// unit from the first microsecond to the last.  Bound: HBM (this card streams 6.1
-// TB/s whatever the order of the rows, as long as whole 128-byte lines are asked for
-// and 48 KB per compute unit are in flight).
+// weights: an expert has few rows (up to about 190 and then one tile, which reads every
+// weight once; in layer calls up to 384, two or three tiles, which run side by side on an
+// XCD), and what counts is that weight bytes are in flight on every compute unit from the
+// first microsecond to the last.  Bound: HBM (this card reads 5.5 to
+// 6.9 TB/s whatever the order of the rows, as long as whole 128-byte lines are asked for
+// and 48 KB per compute unit are in flight; a copy makes 4.8 of reads and writes).
 //
 // One workgroup of eight waves per tile of BM grouped rows x BN weight rows; where
 // the LDS allows it two workgroups per compute unit, one starting up or writing its
@@ -21,12 +22,13 @@
 // so a whole tile gives the same bits whichever kernel multiplies it.
 //
 // Measured, layer call, against the persistent kernels: DiT-XL width, fp16, 512
-// tokens 145 -> 111 us (fc1 65 -> 59, fc2 with the sum of its pieces 68 -> 40; 273 MB
-// of weights: 45 us at the streaming rate); DiT-G width with fp8 weights, 512 tokens
-// 439 -> 255 us (860 MB: 141 us).  What is left over the streaming time: a
-// workgroup's start (row ranges, row table, first copies: 4 to 5 us), the last round
-// of workgroups, and the products, which the lockstep of a workgroup's waves hides
-// only in part.
+// tokens 144 -> 112 us, DiT-G width with fp8 weights, 512 tokens 441 -> 258 us.  Weights and
+// rows in the launches, against that bound: 3.6 TB/s in fc1 (51 us) and 2.9 in fc2 (35 us),
+// fp8 weights 3.75 (153 us) and 3.25 (94 us).  What is left: a workgroup's start (row
+// ranges, row table, first copies: 4 to 5 us), the last round of workgroups (fc2 at 512
+// tokens of DiT-XL width has at most 171 for 256 compute units), and the products, which
+// the lockstep of a workgroup's waves hides only in part: the waves wait for 42 to 49 % of
+// their cycles with the matrix pipe busy for 20 to 32 %.
 //
 // Compiled for bf16 and, through grouped_gemm_stream_f16.hip, for fp16.
 #include <type_traits>

@@ -39,6 +39,12 @@ int launch_stream(const StreamBatch &b, int mode, int act_dtype, hipStream_t s) 
 //   more, GELU: about 185 (1152 wide 239 / 241 at 187; 1408 wide 390 / 384 at 225);
 //   fp8 weights, whose shared expert has launches of its own there: SwiGLU past 288 (DiT-G
 //   width, 2200 tokens 817 / 704), GELU 210 (1600 tokens 608 / 595, 1800 617 / 627).
+// SwiGLU with more than 8 experts has no bound beyond the 192-row tile (about 170 rows per
+// expert), which is too low for 9 and 10 experts (1152 wide, 190 rows per expert, 165 / 147
+// and 157 / 153; 220 rows 157 / 156 and 165 / 169) and too high where the persistent
+// kernels' last turn happens to be full (1152 wide, 12 experts 159 / 133 at 128 rows, 157 / 164
+// at 140; 16 experts 166 / 168 at 100, 197 / 212 at 170; 2048 wide, 16 experts 463 / 460 at 128,
+// 478 / 516 at 170).  No line through rows and experts alone separates these.
 bool stream_pays(int64_t rows, int experts, bool w8, bool gelu, bool shared) {
   if (rows_of_full_expert(rows, experts) <= 192.0) return true;
   if (!shared) return !w8 && experts <= 8 && rows <= 192ll * experts;
@@ -494,7 +500,9 @@ namespace {
 // 142 at 512, 155 / 156 at 768, 164 / 167 at 1024; GELU experts with a shared
 // expert of 2 x the routed width (k = 9216: twice the routed tiles' length) 166 /
 // 116 at 64, 174 / 134 at 512, 216 / 190 at 1024, 241 / 242 at 1536.  The bound
-// on the tile count is the host's (row counts live on the device).
+// on the tile count is the host's (row counts live on the device).  Most of these batches
+// stream now; what is left are a band past the streaming range (4 experts, 770 to 1200
+// tokens at DiT-XL width) and layers that the tuning hook keeps off the streaming kernels.
 bool shared_fc2_alone(const dice_moe_layer_t *L, int64_t n_tokens, int64_t max_rows) {
   const int choice = shared_fc2_launch_choice();
   if (choice != 0) return choice > 0;

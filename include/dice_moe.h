@@ -305,14 +305,18 @@ typedef struct dice_moe_layer {
   int32_t batch_invariant; /* 1: a token's result does not depend on what else is in
                            * the call.  By default an fc2 launch that carries one
                            * problem (fp8 routed weights, no shared expert, or a
-                           * small batch whose shared expert gets its own launch)
+                           * mid-size batch whose shared expert gets its own launch)
                            * and whose tiles leave most workgroups idle in their
                            * last turn cuts that turn's tiles along k and adds the
-                           * 16-bit pieces in fp32 in a fixed order: deterministic,
-                           * but a token's last bit can then depend on the number
-                           * of tokens (or dropped slots) in the call, and a skip
-                           * step fed its own cache need not reproduce the full
-                           * step bit for bit.  1 multiplies every tile whole. */
+                           * 16-bit pieces in fp32 in a fixed order; and small
+                           * batches (16-bit: few rows per expert; fp32: few tiles)
+                           * cut fc2 along k into fp32 partial rows that the combine
+                           * adds up.  Both are deterministic, but a token's last
+                           * bit can then depend on the number of tokens (or
+                           * dropped slots) in the call, and a skip step fed its own
+                           * cache need not reproduce the full step bit for bit.  1
+                           * multiplies every tile whole, and keeps 16-bit layers
+                           * off the kernels for small batches. */
 } dice_moe_layer_t;
 
 /* mode: 0 = plain step; 1 = full step that also writes cache_out ("put");
@@ -463,12 +467,13 @@ int dice_profile_read(float *ms_out, int n);
                                                 * kernel instead of inside it (same results) */
 #define DICE_GEMM_CFG_FC2_WHOLE_TILES 50 /* fc2: no last turn is cut along k (as batch_invariant, for every layer) */
 #define DICE_GEMM_CFG_FC2_SHARED_ALONE 51 /* fc2: the shared expert's fc2 always in a launch of its own */
-#define DICE_GEMM_CFG_FC2_SHARED_JOINT 52 /* fc2: ... never (by default: small batches only) */
+#define DICE_GEMM_CFG_FC2_SHARED_JOINT 52 /* fc2: ... never (by default: a band of mid-size batches only) */
 #define DICE_GEMM_CFG_SLIM_TILES 54      /* either stage: 128-row weight tiles wherever a launch can take them (fc2;
                                             SwiGLU fc1 with gathered rows) */
 #define DICE_GEMM_CFG_NO_SLIM_TILES 55   /* ... never (by default: where the host's model of the workgroups' loads
-                                            says they shorten the launch: fc1 below about 1000 tokens at DiT-XL width,
-                                            fc2 between about 1000 and 2000) */
+                                            says they shorten the launch: fc1 below about 1000 tokens at DiT-XL width
+                                            where the batch does not take the streaming kernels, fc2 between about 1000
+                                            and 2000) */
 int dice_set_gemm_config(int fc1_cfg, int fc2_cfg);
 
 /*
