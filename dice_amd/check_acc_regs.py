@@ -13,6 +13,15 @@ the compiler neither above v127 nor in any accumulation register
 reads the device assembly the compiler wrote for a translation unit and fails
 the build if an instruction outside the inline assembly touches a register that
 belongs to the assembly.
+
+Nor does the compiler know which LDS reads the assembly has left in flight: the
+fragments of the staged kernels (v0 .. v63) are free for it behind the last
+statement of a tile, where the reads of the next tile's first fragments may not
+have landed yet.  So every path from a statement that reads fragments to the
+next full wait for LDS (lgkmcnt(0), in the text or the compiler's own) is
+followed, and an instruction of the compiler on it that names a fragment's
+register fails the build as well: it would read a value that has not arrived, or
+write one that the read then replaces.
 """
 from __future__ import annotations
 
@@ -21,6 +30,8 @@ import sys
 
 _KERNEL = re.compile(r"^(_ZN4dice\S*gemm_persist_kernel(?:4[ad]?|_f8[asd])I\S+):")
 _ANY_FN = re.compile(r"^(\S+):\s*(;.*)?$")
+_LABEL = re.compile(r"^(\.L\w+):")
+_DRAINS = re.compile(r"^s_waitcnt\b.*\blgkmcnt\(0\)")
 _REG = re.compile(r"\b([av])(\d+)\b|\b([av])\[(\d+):(\d+)\]")
 
 
@@ -39,42 +50,113 @@ def _owned_from(mangled: str):
     return (0 if int(m.group(1)) == 256 else 64), 256
 
 
+def _fragments_end(mangled: str) -> int:
+    """The fragments that the assembly reads from LDS are the vector registers below this one (0: not checked)."""
+    return 64 if re.search(r"gemm_persist_kernel(?:4a|_f8a|_f8s)I", mangled) else 0
+
+
+def _registers(code: str):
+    """(file, first, last) of every accumulation or vector register that an instruction names."""
+    for m in _REG.finditer(code):
+        if m.group(1):
+            yield m.group(1), int(m.group(2)), int(m.group(2))
+        else:
+            yield m.group(3), int(m.group(4)), int(m.group(5))
+
+
+def _after_statement(lines):
+    """Whether LDS reads may be in flight behind a statement of the assembly (None: it neither reads nor waits)."""
+    in_flight = None
+    for ln in lines:
+        if ln.startswith("ds_read"):
+            in_flight = True
+        elif _DRAINS.match(ln):
+            in_flight = False
+    return in_flight
+
+
+def _early_touches(body, fragments_end: int):
+    """Instructions of the compiler that name a fragment's register where a read of the assembly may be in flight.
+    `body`: ("label", name), ("asm", lines of a statement) and ("code", instruction) in the order of the text."""
+    label_at = {what: at for at, (kind, what) in enumerate(body) if kind == "label"}
+    work = [at + 1 for at, (kind, what) in enumerate(body) if kind == "asm" and _after_statement(what)]
+    seen, found = set(), set()
+    while work:
+        at = work.pop()
+        while at < len(body) and at not in seen:
+            seen.add(at)
+            kind, what = body[at]
+            at += 1
+            if kind == "asm":
+                if _after_statement(what) is not None:
+                    break                         # it has waited, or its own reads start a path of their own
+            elif kind == "code":
+                if _DRAINS.match(what):
+                    break
+                if any(f == "v" and first < fragments_end for f, first, _ in _registers(what)):
+                    found.add(at - 1)
+                op = what.split()[0]
+                if op in ("s_setpc_b64", "s_swappc_b64"):
+                    raise RuntimeError(f"cannot follow {what}")
+                if op == "s_endpgm":
+                    break
+                if op == "s_branch" or op.startswith("s_cbranch"):
+                    work.append(label_at[what.split()[1]])
+                    if op == "s_branch":
+                        break
+    return [body[at][1] for at in sorted(found)]
+
+
 def check(asm_path: str) -> int:
     """Returns the number of checked kernels; raises on a collision."""
     kernel = None
-    in_asm = False
-    checked = set()
+    statement = None          # lines of the inline assembly being read
+    checked = {}
     problems = []
     with open(asm_path) as f:
         for line in f:
             m = _KERNEL.match(line)
             if m:
                 kernel = m.group(1)
-                checked.add(kernel)
+                checked[kernel] = []
                 continue
             if line.startswith("_Z") and _ANY_FN.match(line):
                 kernel = None
                 continue
+            if kernel is None:
+                continue
+            body = checked[kernel]
             if ";;#ASMSTART" in line:
-                in_asm = True
+                statement = []
                 continue
             if ";;#ASMEND" in line:
-                in_asm = False
+                body.append(("asm", statement))
+                statement = None
                 continue
-            if in_asm or kernel is None or line.startswith("\t."):
+            code = line.split(";")[0].strip()
+            if statement is not None:
+                statement.append(code)
                 continue
-            code = line.split(";")[0]
+            m = _LABEL.match(code)
+            if m:
+                body.append(("label", m.group(1)))
+                continue
+            if not code or code.startswith("."):
+                continue
+            body.append(("code", code))
             first_acc, first_vec = _owned_from(kernel)
-            for m in _REG.finditer(code):
-                if m.group(1):
-                    file_, regs = m.group(1), [int(m.group(2))]
-                else:
-                    file_, regs = m.group(3), range(int(m.group(4)), int(m.group(5)) + 1)
-                if any(r >= (first_acc if file_ == "a" else first_vec) for r in regs):
-                    problems.append(f"{kernel}: {code.strip()}")
+            if any(last >= (first_acc if file_ == "a" else first_vec) for file_, _, last in _registers(code)):
+                problems.append(f"{kernel}: {code}")
     if problems:
         raise RuntimeError(
             "the compiler placed values of its own in registers that belong to the kernel's assembly "
+            f"({len(problems)} instructions), e.g.\n  " + "\n  ".join(problems[:8]))
+    for kernel, body in checked.items():
+        if _fragments_end(kernel):
+            problems += [f"{kernel}: {code}" for code in _early_touches(body, _fragments_end(kernel))]
+    if problems:
+        raise RuntimeError(
+            "the compiler uses registers of fragments whose LDS reads may still be in flight "
             f"({len(problems)} instructions), e.g.\n  " + "\n  ".join(problems[:8]))
     if not checked:
         raise RuntimeError(f"{asm_path}: no checked kernel found")

@@ -397,8 +397,7 @@ __device__ __forceinline__ void gemm_persist_f8_asm_body(const PersistBatch &bat
       advance_copy();
       DICE_F8_STEP(d_s1, LIVE);
     }
-    // The last reads (of the next tile, which reads them again: the epilogue needs the registers) have landed.
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+{v[0:31]}"(f0), "+{v[32:63]}"(f1)::"memory");
+    // (its last reads are waited for where the four forms of this loop have met)
   };
 
   auto run_tile = [&](auto live_c) {
@@ -411,6 +410,16 @@ __device__ __forceinline__ void gemm_persist_f8_asm_body(const PersistBatch &bat
     else if (live == 3) run_tile(template_int<3>{});
     else if (live == 2) run_tile(template_int<2>{});
     else run_tile(template_int<1>{});
+    if constexpr (!DMA) {
+      // The last reads (of the next tile, which reads them again: the epilogue needs their registers) have landed.
+      // (One wait behind the four loops, not one that names the fragments at the end of each: with those the
+      // compiler kept the scalars that the loops carry in vector registers, which the text's loads cannot take.
+      // The fences keep the epilogue's first instructions, which name v0 as soon as they may, behind it;
+      // check_acc_regs.py looks for any that got in front.)
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    }
     fixed_acc_settle();
     // (behind the epilogue's stores, which retire in another order, a count would not tell the copies apart)
     if constexpr (DMA && BLK == 1) pwait_vmcnt<0>();

@@ -263,3 +263,37 @@ def test_register_check_flags_compiler_code_in_the_assemblys_registers(tmp_path)
     path.write_text("_Z5otherv:\n\ts_endpgm\n")
     with pytest.raises(RuntimeError, match="no checked kernel"):
         check(str(path))
+
+
+@pytest.mark.parametrize("name", ["121gemm_persist_kernel4aILi0ELi256ELb1ELb1ELb0E", "123gemm_persist_kernel_f8aILi0ELb0ELb0E",
+                                  "123gemm_persist_kernel_f8sILb1E"])
+def test_register_check_flags_fragments_used_before_their_reads_landed(tmp_path, name):
+    """Between a statement that reads fragments and the wait for them (a statement's, or the compiler's
+    own) no compiled instruction may name a fragment's register, on any path."""
+    from dice_amd.check_acc_regs import check
+    kernel = f"_ZN4dice12_GLOBAL__N_{name}EvNS_12PersistBatchE"
+    loop = [".LBB0_1:", "\t;;#ASMSTART", "\ts_waitcnt lgkmcnt(0)", "\tds_read_b128 v[28:31], v70 offset:64",
+            "\ts_waitcnt lgkmcnt(3)", "\t;;#ASMEND", "\ts_add_i32 s4, s4, 2"]
+    wait = ["\t;;#ASMSTART", "\ts_waitcnt lgkmcnt(0)", "\t;;#ASMEND"]
+    touch, elsewhere = ["\tv_cvt_f32_u32_e32 v0, s92"], ["\tv_mov_b32_e32 v64, v65"]
+    again = ["\ts_cbranch_scc1 .LBB0_1"]
+    ok = [
+        loop + again + elsewhere + wait + touch,
+        loop + again + ["\ts_waitcnt vmcnt(0) lgkmcnt(0)"] + touch,              # the compiler's own wait will do
+        touch + loop + again + ["\ts_branch .LBB0_3", ".LBB0_2:"] + touch + ["\ts_endpgm", ".LBB0_3:"] + wait + touch,
+    ]
+    bad = [
+        loop + again + touch + wait,
+        loop + again + ["\ts_waitcnt lgkmcnt(1)"] + touch + wait,                # (a count says nothing about these reads)
+        loop + ["\ts_cbranch_vccz .LBB0_3"] + again + wait + ["\ts_endpgm", ".LBB0_3:"] + touch + wait,
+        loop + touch + again + wait,
+        loop + again + ["\tds_read_b128 v[60:63], v90"] + wait,
+    ]
+    path = tmp_path / "k.s"
+    for lines in ok:
+        path.write_text(_fake_asm(kernel, lines))
+        assert check(str(path)) == 1
+    for lines in bad:
+        path.write_text(_fake_asm(kernel, lines))
+        with pytest.raises(RuntimeError, match="may still be in flight"):
+            check(str(path))
