@@ -3,10 +3,17 @@
 ``python -m dice_amd.build`` (or ``build_library()``) cross-compiles without a
 GPU.  Objects go to ``dice_amd/_build/``; the shared library stays in-tree next
 to this file so it travels with the source tree.
+
+Every object of the library names the digest of the sources and flags that it was
+compiled from (csrc/built_from.h); ``lib.load()`` refuses a library of which any
+object's differs from that of the sources beside it.
 """
 from __future__ import annotations
 
+import glob
+import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -14,6 +21,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
+INCLUDE = os.path.join(HERE, "..", "include")
 BUILD_DIR = os.path.join(HERE, "_build")
 LIB_PATH = os.path.join(HERE, "libdice_moe.so")
 
@@ -47,6 +55,33 @@ HIP_FLAGS = [
 ]
 
 
+def source_digest(csrc: str = CSRC, include: str = INCLUDE):
+    """Digest of everything a build reads: kernels, headers, generators and flags.  None where the sources are not
+    there to build from (a copy of the package without them)."""
+    paths = sorted(p for pat in ("*.hip", "*.h", "*.py") for p in glob.glob(os.path.join(csrc, pat)))
+    headers = sorted(glob.glob(os.path.join(include, "*.h")))
+    if not paths or not headers:
+        return None
+    h = hashlib.sha256("\0".join(HIP_FLAGS + SOURCES).encode())
+    for path in paths + headers:
+        with open(path, "rb") as f:
+            data = f.read()
+        h.update(f"\0{os.path.basename(path)}\0{len(data)}\0".encode())
+        h.update(data)
+    return h.hexdigest()
+
+
+_BUILT_FROM = re.compile(rb"dice_moe unit (\S+) ([0-9a-f]{64})\0")
+
+
+def stale_units(library: bytes, digest: str):
+    """The sources whose object in a library (its bytes) is missing or was compiled from anything but `digest`."""
+    found = {}
+    for m in _BUILT_FROM.finditer(library):
+        found.setdefault(m.group(1).decode(), set()).add(m.group(2).decode())
+    return [s for s in SOURCES if found.get(s) != {digest}]
+
+
 def _hipcc() -> str:
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(exe):
@@ -75,10 +110,17 @@ def _generate_sources() -> None:
                 f.write(text)
 
 
-def _compile(src: str, extra) -> str:
+def _remove(path: str) -> None:
+    if os.path.exists(path):
+        os.remove(path)
+
+
+def _compile(src: str, extra, digest: str) -> str:
     stem = os.path.splitext(src)[0]
     obj = os.path.join(BUILD_DIR, stem + ".o")
-    cmd = [_hipcc(), *HIP_FLAGS, "-I", BUILD_DIR, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+    _remove(obj)                  # (a source that no longer compiles leaves no object of an older one behind)
+    cmd = [_hipcc(), *HIP_FLAGS, "-I", BUILD_DIR, f'-DDICE_BUILT_FROM="dice_moe unit {src} {digest}"',
+           "-include", os.path.join(CSRC, "built_from.h"), *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     if src in ACC_CHECKED:
         cmd.insert(-4, "-save-temps=obj")
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -86,7 +128,11 @@ def _compile(src: str, extra) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")
     if src in ACC_CHECKED:
         from dice_amd.check_acc_regs import check
-        check(os.path.join(BUILD_DIR, stem + "-hip-amdgcn-amd-amdhsa-gfx950.s"))
+        try:
+            check(os.path.join(BUILD_DIR, stem + "-hip-amdgcn-amd-amdhsa-gfx950.s"))
+        except RuntimeError:
+            _remove(obj)
+            raise
     return obj
 
 
@@ -95,11 +141,13 @@ def build_library(verbose: bool = True, extra_flags=(), out: str = None) -> str:
     package's own path when given: a second build to compare with, e.g.
     ``python -m dice_amd.build --out /tmp/other.so -DDICE_MFMA_ROWS_OUTERMOST=1``)."""
     target = os.path.abspath(out) if out else LIB_PATH
+    _remove(target)               # (a build that fails leaves no library, rather than the one before)
     os.makedirs(BUILD_DIR, exist_ok=True)
+    digest = source_digest()      # (before the compiler reads anything: a source edited meanwhile makes its object stale)
     _generate_sources()
     jobs = min(len(SOURCES), max(1, min(8, os.cpu_count() or 1)))
     with ThreadPoolExecutor(jobs) as pool:
-        objs = list(pool.map(lambda s: _compile(s, list(extra_flags)), SOURCES))
+        objs = list(pool.map(lambda s: _compile(s, list(extra_flags), digest), SOURCES))
     tmp = target + ".tmp"
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -1,7 +1,8 @@
 """ctypes binding of ``libdice_moe.so`` (the C ABI declared in include/dice_moe.h).
 
 The library is the product path.  There is no CPU or eager-torch fallback: if
-the shared object is missing or a call fails, an exception is raised.
+the shared object is missing, was built from other sources than those beside it,
+or a call fails, an exception is raised.
 """
 from __future__ import annotations
 
@@ -107,6 +108,14 @@ def load() -> ctypes.CDLL:
         raise DiceError(
             f"{LIB_PATH} is missing: build it with `python -m dice_amd.build` "
             "(there is no fallback path)")
+    from .build import source_digest, stale_units
+    digest = source_digest()
+    if digest is not None:
+        with open(LIB_PATH, "rb") as f:
+            stale = stale_units(f.read(), digest)
+        if stale:
+            raise DiceError(f"{LIB_PATH} was built from other sources than those beside it ({', '.join(stale)}): "
+                            "build it again with `python -m dice_amd.build`")
     lib = ctypes.CDLL(LIB_PATH)
     lib.dice_abi_version.restype = c_int
     lib.dice_last_error.restype = c_char_p
