@@ -14,14 +14,17 @@ reads the device assembly the compiler wrote for a translation unit and fails
 the build if an instruction outside the inline assembly touches a register that
 belongs to the assembly.
 
-Nor does the compiler know which LDS reads the assembly has left in flight: the
-fragments of the staged kernels (v0 .. v63) are free for it behind the last
-statement of a tile, where the reads of the next tile's first fragments may not
-have landed yet.  So every path from a statement that reads fragments to the
-next full wait for LDS (lgkmcnt(0), in the text or the compiler's own) is
-followed, and an instruction of the compiler on it that names a fragment's
-register fails the build as well: it would read a value that has not arrived, or
-write one that the read then replaces.
+Nor does the compiler know which LDS reads the assembly has left in flight.  The
+staged kernels (fragments in v0 .. v63) leave a tile's last statement with reads of
+the next tile's first fragments under way, and those that copy straight to LDS
+(gemm_persist_kernel4d, gemm_persist_kernel_f8d: v0 .. v127) also run compiled
+code - a whole tile switch - between the two statements of every step with those
+of the second k-block under way.  A value moved out of such a register has not
+arrived yet, one put there is overwritten when it does.  So every path from a
+statement that reads fragments to the next statement that waits for all of LDS
+(lgkmcnt(0)) is followed, and an instruction of the compiler on it that names a
+fragment's register fails the build as well.  (Its own waits do not end a path:
+the fragments are the assembly's for the whole k-loop.)
 """
 from __future__ import annotations
 
@@ -39,7 +42,7 @@ def _owned_from(mangled: str):
     """(first accumulation register, first vector register) the assembly owns."""
     if "gemm_persist_kernel4aI" in mangled or "gemm_persist_kernel_f8aI" in mangled:
         return 0, 128
-    if "gemm_persist_kernel4dI" in mangled or "gemm_persist_kernel_f8dI" in mangled:   # (no operand data waits in vector registers there)
+    if "gemm_persist_kernel4dI" in mangled or "gemm_persist_kernel_f8dI" in mangled:   # (no vector register is the text's for good)
         return 0, 256
     if "gemm_persist_kernel_f8sI" in mangled:     # the scaled kind's text also names v117 .. v127
         return 0, 117
@@ -52,6 +55,8 @@ def _owned_from(mangled: str):
 
 def _fragments_end(mangled: str) -> int:
     """The fragments that the assembly reads from LDS are the vector registers below this one (0: not checked)."""
+    if re.search(r"gemm_persist_kernel(?:4d|_f8d)I", mangled):
+        return 128
     return 64 if re.search(r"gemm_persist_kernel(?:4a|_f8a|_f8s)I", mangled) else 0
 
 
@@ -76,7 +81,7 @@ def _after_statement(lines):
 
 
 def _early_touches(body, fragments_end: int):
-    """Instructions of the compiler that name a fragment's register where a read of the assembly may be in flight.
+    """Instructions of the compiler that name a fragment's register between a statement that reads and one that waits.
     `body`: ("label", name), ("asm", lines of a statement) and ("code", instruction) in the order of the text."""
     label_at = {what: at for at, (kind, what) in enumerate(body) if kind == "label"}
     work = [at + 1 for at, (kind, what) in enumerate(body) if kind == "asm" and _after_statement(what)]
@@ -91,8 +96,6 @@ def _early_touches(body, fragments_end: int):
                 if _after_statement(what) is not None:
                     break                         # it has waited, or its own reads start a path of their own
             elif kind == "code":
-                if _DRAINS.match(what):
-                    break
                 if any(f == "v" and first < fragments_end for f, first, _ in _registers(what)):
                     found.add(at - 1)
                 op = what.split()[0]

@@ -265,29 +265,32 @@ def test_register_check_flags_compiler_code_in_the_assemblys_registers(tmp_path)
         check(str(path))
 
 
-@pytest.mark.parametrize("name", ["121gemm_persist_kernel4aILi0ELi256ELb1ELb1ELb0E", "123gemm_persist_kernel_f8aILi0ELb0ELb0E",
-                                  "123gemm_persist_kernel_f8sILb1E"])
-def test_register_check_flags_fragments_used_before_their_reads_landed(tmp_path, name):
-    """Between a statement that reads fragments and the wait for them (a statement's, or the compiler's
-    own) no compiled instruction may name a fragment's register, on any path."""
+@pytest.mark.parametrize("name,end", [("121gemm_persist_kernel4aILi0ELi256ELb1ELb1ELb0E", 64),
+                                      ("123gemm_persist_kernel_f8aILi0ELb0ELb0E", 64),
+                                      ("123gemm_persist_kernel_f8sILb1E", 64),
+                                      ("121gemm_persist_kernel4dILi0ELi256ELb1ELb0E", 128),
+                                      ("123gemm_persist_kernel_f8dILi0ELb0ELb0E", 128)])
+def test_register_check_flags_fragments_used_before_their_reads_landed(tmp_path, name, end):
+    """Between a statement that reads fragments and the statement that waits for them no compiled
+    instruction may name a fragment's register, on any path."""
     from dice_amd.check_acc_regs import check
     kernel = f"_ZN4dice12_GLOBAL__N_{name}EvNS_12PersistBatchE"
     loop = [".LBB0_1:", "\t;;#ASMSTART", "\ts_waitcnt lgkmcnt(0)", "\tds_read_b128 v[28:31], v70 offset:64",
             "\ts_waitcnt lgkmcnt(3)", "\t;;#ASMEND", "\ts_add_i32 s4, s4, 2"]
     wait = ["\t;;#ASMSTART", "\ts_waitcnt lgkmcnt(0)", "\t;;#ASMEND"]
-    touch, elsewhere = ["\tv_cvt_f32_u32_e32 v0, s92"], ["\tv_mov_b32_e32 v64, v65"]
+    touch, elsewhere = [f"\tv_cvt_f32_u32_e32 v{end - 1}, s92"], [f"\tv_add_u32_e32 v{end}, 4, v{end}"]
     again = ["\ts_cbranch_scc1 .LBB0_1"]
     ok = [
         loop + again + elsewhere + wait + touch,
-        loop + again + ["\ts_waitcnt vmcnt(0) lgkmcnt(0)"] + touch,              # the compiler's own wait will do
         touch + loop + again + ["\ts_branch .LBB0_3", ".LBB0_2:"] + touch + ["\ts_endpgm", ".LBB0_3:"] + wait + touch,
     ]
     bad = [
         loop + again + touch + wait,
+        loop + elsewhere + touch + loop[1:] + again + wait,                      # (compiled code between two statements of a step)
         loop + again + ["\ts_waitcnt lgkmcnt(1)"] + touch + wait,                # (a count says nothing about these reads)
         loop + ["\ts_cbranch_vccz .LBB0_3"] + again + wait + ["\ts_endpgm", ".LBB0_3:"] + touch + wait,
         loop + touch + again + wait,
-        loop + again + ["\tds_read_b128 v[60:63], v90"] + wait,
+        loop + again + [f"\tds_read_b128 v[{end - 1}:{end + 2}], v{end + 6}"] + wait,
     ]
     path = tmp_path / "k.s"
     for lines in ok:
