@@ -26,8 +26,8 @@ tile.  The second statement opens with the workgroup barrier; block D then
 reads the first fragments of step s + 1, writes quarter 0 of stage S (step
 s + 2) to slot S and refills it with quarter 0 of step s + 4.
 
-Kinds 0, 1, 4, 5, 6 are the 16-bit shapes (SwiGLU fc1 on 256 weight rows, fc2 on 192
-and on 128, GELU fc1 on 256, SwiGLU fc1 on 128).  Kinds 2 and 3 are the kernel for fp8 activations and weights
+Kinds 0, 1 and 5 are the 16-bit shapes (SwiGLU fc1 on 256 weight rows, fc2 on 192,
+GELU fc1 on 256).  Kinds 2 and 3 are the kernel for fp8 activations and weights
 (grouped_gemm_persist_f8.hip): the same stages, slots and quarters, but a step
 is 128 k in two k-blocks of 64, a fragment is 32 bytes per lane (two LDS reads)
 and there is one set of eight fragments in v[0:63] (weight block j at 8 j, row
@@ -64,9 +64,7 @@ KINDS = {
     # kind: (TN, copies of B per step, B frag row offsets (rows), acc block 0, B loads that use the second descriptor)
     0: dict(name="fc1 SwiGLU, 256 weight rows", TN=4, CB=8, brow=[0, 32, 128, 160], acc0=0, up_from=4),
     1: dict(name="fc2, 192 weight rows", TN=3, CB=6, brow=[0, 32, 64], acc0=4, up_from=99),
-    4: dict(name="fc2, 128 weight rows", TN=2, CB=4, brow=[0, 32], acc0=8, up_from=99),
     5: dict(name="GELU fc1, 256 weight rows", TN=4, CB=8, brow=[0, 32, 64, 96], acc0=0, up_from=99),
-    6: dict(name="fc1 SwiGLU, 128 weight rows", TN=2, CB=4, brow=[0, 64], acc0=8, up_from=2),
     # fp8 activations and weights (grouped_gemm_persist_f8.hip): a step is 128 k in two halves of 64 k
     2: dict(name="fp8 SwiGLU fc1, 256 weight rows", TN=4, CB=8, brow=[0, 32, 128, 160], acc0=0, up_from=4, f8=True),
     3: dict(name="fp8 GELU fc1 / fc2, 256 weight rows", TN=4, CB=8, brow=[0, 32, 64, 96], acc0=0, up_from=99, f8=True),
@@ -328,12 +326,10 @@ class Stream:
         quarter q of stage wstage to its slot, then refilled."""
         tn, cb = self.k["TN"], self.k["CB"]
         prods = [(i, ((tn - 1 - m) if (i & 1) else m)) for i in range(self.live) for m in range(tn)]
-        if var == 2:
-            prods = []
         reads = self.frag_order()
         f, e = self.qfirst(q), self.qfirst(q + 1)
         items = list(range(f, e))
-        mf = max(1, len(prods))
+        mf = len(prods)
         gaps = [[] for _ in range(mf)]
         for n, r in enumerate(reads):
             gaps[side_slot(n, len(reads), mf, 0)].append(("r", r))
@@ -342,9 +338,8 @@ class Stream:
         for n, l in enumerate(items):
             gaps[side_slot(n, len(items), mf, 3)].append(("l", l))
         for g in range(mf):
-            if prods:
-                i, j = prods[g]
-                self.mfma(mbuf, i, j, var == 1)
+            i, j = prods[g]
+            self.mfma(mbuf, i, j, var == 1)
             # reads first: a read queued behind a write waits for the write's 16 cycles
             for kind in ("r", "w", "l"):
                 for k2, x in gaps[g]:
@@ -361,10 +356,10 @@ class Stream:
         if self.k.get("f8"):
             return self.abc8(slot, var)
         self.block(0, slot, 1, slot ^ 1, 1, var)
-        self.block(1, slot, 2, slot ^ 1, 2, 0 if var == 1 else var)
-        self.block(0, slot, 3, slot ^ 1, 3, 0 if var == 1 else var)
+        self.block(1, slot, 2, slot ^ 1, 2, 0)
+        self.block(0, slot, 3, slot ^ 1, 3, 0)
 
-    def d(self, slot, var):
+    def d(self, slot):
         if self.k.get("f8"):
             return self.d8(slot)
         # This wave has read slot `slot` for the last time and finished writing the other one;
@@ -374,7 +369,7 @@ class Stream:
         self.needed.add((self.key, self.site))
         self.wait("lgkm", self.lds_issued)
         self.emit("s_barrier")
-        self.block(1, slot ^ 1, 0, slot, 0, 0 if var == 1 else var)
+        self.block(1, slot ^ 1, 0, slot, 0, 0)
 
     def load_step(self, stage):
         for l in range(self.n_loads()):
@@ -443,7 +438,7 @@ def simulate(kind, live):
             slot = s & 1
             var = 1 if s == 0 else 0
             rec(f"abc_s{slot}_v{var}", st.abc, slot, var)
-            rec(f"d_s{slot}", st.d, slot, 0)
+            rec(f"d_s{slot}", st.d, slot)
         # the epilogue: LDS traffic of the host code, drained; vector loads stay in flight
         st.lds_done = st.lds_issued
     # the variant of a first step whose sums do not start from zero (biased tiles) is the plain one: v0 of slot 0

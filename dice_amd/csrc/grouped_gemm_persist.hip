@@ -784,32 +784,33 @@ __device__ __forceinline__ void gemm_persist64_body(const PersistBatch &batch) {
 // Taken for launches of 16-bit weights that rewrite the tile table (the others take
 // gemm_persist_dma_body, which has no variant that does).
 
-template <int MODE, bool HAS_BIAS, int BN, bool GATHER, bool W8>
+// (SwiGLU fc1 on 256 weight rows, whose activation rows may be addressed through a row table; GELU fc1 on 256; fc2
+// on 192 without a bias.)
+template <int MODE, bool HAS_BIAS, int BN, bool GATHER>
 constexpr bool persist64_asm_applies() {
-  return !W8 && ((!HAS_BIAS && MODE == kFc1Swiglu && (BN == 256 || BN == 128) && GATHER) || (!HAS_BIAS && MODE == kFc2 && BN == 192) ||
-                 (MODE == kFc2 && BN == 128) || (MODE == kFc1Gelu && BN == 256));
+  return (!HAS_BIAS && MODE == kFc1Swiglu && BN == 256 && GATHER) || (!HAS_BIAS && MODE == kFc2 && BN == 192) ||
+         (MODE == kFc1Gelu && BN == 256);
 }
 
-// HAS_BIAS (fc2 on 128-row weight tiles and GELU fc1, whose staging rows leave room for it):
-// the tile's bias is staged in LDS a tile ahead, as the fp8 kernel does, and added in the epilogue.
-template <int MODE, int BN, bool GATHER, bool REFILL, bool HAS_BIAS = false>
+// HAS_BIAS (GELU fc1, whose staging rows leave room for it): the tile's bias is staged in LDS a tile ahead, as the
+// fp8 kernel does, and added in the epilogue.
+template <int MODE, bool HAS_BIAS>
 __device__ __forceinline__ void gemm_persist64_asm_body(const PersistBatch &batch) {
-  constexpr bool SWIGLU = MODE == kFc1Swiglu;
-  constexpr int KIND = SWIGLU ? (BN == 256 ? 0 : 6) : MODE == kFc1Gelu ? 5 : BN == 192 ? 1 : 4;
-  static_assert(SWIGLU ? (BN == 256 || BN == 128) : MODE == kFc1Gelu ? BN == 256 : (BN == 192 || BN == 128),
-                "the shapes the generator writes");
+  static_assert(!HAS_BIAS || MODE == kFc1Gelu, "no LDS for a staged bias beside these staging rows");
+  constexpr bool SWIGLU = MODE == kFc1Swiglu, GATHER = SWIGLU;
+  constexpr int BN = MODE == kFc2 ? 192 : 256;
+  constexpr int KIND = SWIGLU ? 0 : MODE == kFc1Gelu ? 5 : 1;   // of gen_persist64_asm.py
   constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
   constexpr int WTN = BN / 2, TM = 4, TN = WTN / 32;
   constexpr int kCopiesA = kPBM / 8 / kQWaves, kCopiesB = BN / 8 / kQWaves;
   constexpr int kAccBlock0 = 16 - TM * TN;
-  static_assert(!HAS_BIAS || (BN == 128 && !GATHER) || MODE == kFc1Gelu, "no LDS for a staged bias beside these staging rows");
   constexpr int kTableBytes = kTableTurns * kTileWords * 4, kRowSlotBytes = kPBM * 4;
   // (three bias buffers: the epilogue of a tile reads its bias while the first wave, a little ahead, may already
   // stage that of the tile after the next)
   constexpr int kBiasBufFloats = 256, kBiasBytes = HAS_BIAS ? 3 * kBiasBufFloats * 4 : 0;
   constexpr int kEpiReserve = kTableBytes + (GATHER ? kRowSlotBytes : 0) + kBiasBytes;
   // (what the epilogue's staging rows must leave free: passed on where it decides the height of a band)
-  constexpr int kReserveArg = HAS_BIAS || MODE == kFc1Gelu ? kEpiReserve : 0;
+  constexpr int kReserveArg = MODE == kFc1Gelu ? kEpiReserve : 0;
   using Epi = EpiGeom<MODE, kQWaves, TM, TN, kReserveArg>;
   typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
 
@@ -832,16 +833,14 @@ __device__ __forceinline__ void gemm_persist64_asm_body(const PersistBatch &batc
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   phase_barrier();
   auto fetch_tile = [&](int turn) {
-    if constexpr (REFILL) {
-      if (turn != 0 && (turn & (kTableTurns - 1)) == 0) {
-        phase_barrier();
-        if (wave == 0) {
-          TileWalker<BN_OUT> walk(batch, lane);
-          walk.build_table(batch, lane, kQBK, tile_table, false, turn);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        phase_barrier();
+    if (turn != 0 && (turn & (kTableTurns - 1)) == 0) {
+      phase_barrier();
+      if (wave == 0) {
+        TileWalker<BN_OUT> walk(batch, lane);
+        walk.build_table(batch, lane, kQBK, tile_table, false, turn);
       }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      phase_barrier();
     }
     int lane_c = lane;   // (opaque: worked out at the tile switch, not held through the k-loop)
     asm volatile("" : "+v"(lane_c));
@@ -1073,10 +1072,10 @@ __global__ __launch_bounds__(4 * kWave, 1) void gemm_persist_kernel4(PersistBatc
 // The same with the k-loop in assembly (gemm_persist64_asm_body).  The compiler
 // allocates from v0..v127 only; v128..v255 and every accumulation register
 // belong to the assembly text.
-template <int MODE, int BN, bool GATHER, bool REFILL = false, bool HAS_BIAS = false>
+template <int MODE, bool HAS_BIAS>
 __global__ __launch_bounds__(4 * kWave, 1) __attribute__((amdgpu_num_vgpr(128)))
 void gemm_persist_kernel4a(PersistBatch batch) {
-  gemm_persist64_asm_body<MODE, BN, GATHER, REFILL, HAS_BIAS>(batch);
+  gemm_persist64_asm_body<MODE, HAS_BIAS>(batch);
 }
 // Operands copied straight to LDS, products of 16 x 16 x 32 (gemm_persist_dma_body).  Every accumulation
 // register belongs to the text.
@@ -1230,15 +1229,15 @@ PersistKernel pick64(bool w8, bool refill) {
       return refill ? gemm_persist_kernel4<MODE, HAS_BIAS, BN, GATHER, true, true>
                     : gemm_persist_kernel4<MODE, HAS_BIAS, BN, GATHER, true, false>;
   }
-  if constexpr (persist_dma_applies<MODE, HAS_BIAS, BN, GATHER, false>()) {
+  if constexpr (persist_dma_applies<MODE, HAS_BIAS, BN, GATHER>()) {
     // (SwiGLU launches without a row table take the instantiation that can have one)
     if (!refill) return gemm_persist_kernel4d<MODE, BN, GATHER || MODE == kFc1Swiglu, HAS_BIAS>;
   }
   if constexpr (MODE == kFc1Gelu && GATHER)   // (only launches that fit the tile table: persist64_ok)
     return nullptr;
-  else if constexpr (persist64_asm_applies<MODE, HAS_BIAS, BN, GATHER, false>())
-    return gemm_persist_kernel4a<MODE, BN, GATHER, true, HAS_BIAS>;
-  else if constexpr (persist_dma_applies<MODE, HAS_BIAS, BN, GATHER, false>())
+  else if constexpr (persist64_asm_applies<MODE, HAS_BIAS, BN, GATHER>())
+    return gemm_persist_kernel4a<MODE, HAS_BIAS>;
+  else if constexpr (persist_dma_applies<MODE, HAS_BIAS, BN, GATHER>())
     return gemm_persist_kernel4<MODE, HAS_BIAS, BN, GATHER, false, true>;
   else
     return refill ? gemm_persist_kernel4<MODE, HAS_BIAS, BN, GATHER, false, true>

@@ -176,9 +176,9 @@ __device__ __forceinline__ void dma_epilogue(const Tile &cp, unsigned char *stag
 }
 
 // The tile shapes the generator writes.  GATHER: activation rows may be addressed through a row table.
-template <int MODE, bool HAS_BIAS, int BN, bool GATHER, bool W8>
+template <int MODE, bool HAS_BIAS, int BN, bool GATHER>
 constexpr bool persist_dma_applies() {
-  if (W8 || (GATHER && MODE == kFc2)) return false;
+  if (GATHER && MODE == kFc2) return false;
   if (MODE == kFc1Swiglu) return !HAS_BIAS && (BN == 256 || BN == 128);
   if (MODE == kFc1Gelu) return BN == 256;
   return BN == 192 || BN == 128 || (BN == 256 && !HAS_BIAS);
@@ -187,7 +187,7 @@ constexpr bool persist_dma_applies() {
 // HAS_BIAS: the tile's bias is staged in LDS a tile ahead and added in the epilogue.
 template <int MODE, int BN, bool GATHER, bool HAS_BIAS>
 __device__ __forceinline__ void gemm_persist_dma_body(const PersistBatch &batch) {
-  static_assert(persist_dma_applies<MODE, HAS_BIAS, BN, GATHER, false>(), "the shapes the generator writes");
+  static_assert(persist_dma_applies<MODE, HAS_BIAS, BN, GATHER>(), "the shapes the generator writes");
   constexpr bool SWIGLU = MODE == kFc1Swiglu;
   constexpr int KIND = SWIGLU ? (BN == 256 ? 0 : 4) : BN == 256 ? 3 : BN == 192 ? 1 : 2;
   constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
