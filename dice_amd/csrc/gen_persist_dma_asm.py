@@ -1,6 +1,6 @@
 """Generates ``persist_dma_asm.inc``: the k-loop of the expert GEMM kernels whose
 operands go from memory straight to LDS (gemm_persist_dma_body in csrc/persist_dma.h,
-gemm_persist_f8_dma_body in csrc/grouped_gemm_persist_f8.hip), as inline assembly on
+gemm_persist_f8_asm_body in csrc/grouped_gemm_persist_f8.hip), as inline assembly on
 fixed registers.
 
 Two things set it apart from the loop of gen_persist64_asm.py, which stages operands
