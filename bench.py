@@ -638,7 +638,8 @@ def measure(cfg_name, variant, activations, dev, steps, warmup, stages=True):
     swiglu = variant == "swiglu"
     if fc1_ms > 0:
         ach = dom_flops / (fc1_ms * 1e-3) / 1e12
-        kern = ("gemm_persist_kernel_f8" if a8 else "gemm_persist_kernel4") if cfg["dtype"] != "f32" else "grouped_gemm_f32_kernel"
+        kern = ("grouped_gemm_split_kernel" if cfg["dtype"] == "f32" else "gemm_persist_kernel_f8d" if a8
+                else "gemm_persist_kernel4" if cfg.get("fp8") else "gemm_persist_kernel4d")
         res["roofline"] = {"bound": "mfma",
                            "kernel": "%s<fc1 %s> (routed%s fc1, activation fused)"
                                      % (kern, "SwiGLU" if swiglu else "GELU-tanh, biased", " + shared expert" if joint else ""),
